@@ -354,6 +354,37 @@ constexpr int share_unroll(int wmax, int frag_in_bytes) {
   return clamp_unroll(kReduceLoadBytesPerLane / (wmax * frag_in_bytes));
 }
 
+// Waves per CU of the W-way reductions.  A CU holds 32 one-wave workgroups, and
+// with all 32 in flight these kernels move less than the memory can: 67 MB of
+// requests to W + 3 streams are queued at once, in an order in which the DRAM
+// finds few open rows.  Fewer waves in flight keep the requests of a moment
+// closer together in every stream (workgroups start in grid order), so each
+// dispatch asks for LDS it never touches, as much as leaves room for the number
+// of workgroups below on a CU.  Measured on MI355X, GB/s at 32 / 18 / 16 / 12 /
+// 10 / 8 waves per CU, on the real tables (GPT-2-124M fp32 W = 8, GPT-2-medium
+// bf16 W = 4, four Llama-7B layers bf16 into fp32 W = 8, GPT-2-124M fp16 W = 8):
+//   fp32         6171 / 6243 / 6297 / 6467 / 6470 / 6290
+//   bf16         6346 / 6576 / 6579 / 6103 / 5600 / 4984
+//   bf16 -> fp32 5927 / 6151 / 6234 / 6152 / 5939 / 5303
+//   fp16         6057 / 6094 / 6186 / 6090 / 5556 / --
+// The lower end is where the waves' own instructions are no longer hidden: the
+// 16-bit types need more of them per byte.  (Copies, with one load and one store
+// per lane, lose from 25 waves down and are launched without a bound.)
+constexpr int kCus = 256;
+constexpr int kLdsBytesPerCu = 160 * 1024;
+constexpr int kLdsGranule = 1280;  // a workgroup's LDS is allocated in these
+// LDS bytes that leave room for `waves` one-wave workgroups on a CU.
+constexpr int lds_for_waves(int waves) { return kLdsBytesPerCu / waves / kLdsGranule * kLdsGranule; }
+constexpr int reduce_waves(int in_size, int world) { return in_size == 4 ? (world <= 4 ? 12 : 10) : 16; }
+// The bound pays once a CU gets several times the workgroups it holds; a short
+// dispatch is over before the queues are full, and its start and end take longer
+// with fewer waves (13.5K workgroups, fp32 W = 4: 17.5 us unbounded, 17.2 at 18
+// waves, 17.7 at 12; 7.5K workgroups, a share of 77 MB: 16.4, 16.5 at 16, 17.0 at 12).
+inline int reduce_lds(int blocks, int waves) {
+  if (blocks < 32 * kCus) return 0;
+  return lds_for_waves(blocks < 128 * kCus ? max_size(waves, 18) : waves);
+}
+
 // Non-SUM all-reduce (mdx_allreduce_op): runs of the replica layout in the
 // kernel arguments, one-wave workgroups.  A lane takes op_unroll(WMAX)
 // 16-byte vectors of every replica -- about 128 bytes of loads in flight, as

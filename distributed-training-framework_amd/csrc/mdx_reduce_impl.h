@@ -278,8 +278,9 @@ struct ArgAllreduce {
   const PieceBatch& b;
   template <int W>
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
-    hipLaunchKernelGGL((allreduce_kernel<T, G, W, UNPACK>), dim3(b.first_block[b.count]), dim3(kBlock), 0,
-                       stream, b, p);
+    const int blocks = b.first_block[b.count];
+    hipLaunchKernelGGL((allreduce_kernel<T, G, W, UNPACK>), dim3(blocks), dim3(kBlock),
+                       reduce_lds(blocks, reduce_waves(sizeof(T), W)), stream, b, p);
     return hipGetLastError();
   }
 };
@@ -291,7 +292,8 @@ struct DevAllreduceUnpack {
   template <int W>
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
-      hipLaunchKernelGGL((allreduce_unpack_kernel_dev<T, G, W>), dim3(grid), dim3(kBlock), 0, stream, slice, p);
+      hipLaunchKernelGGL((allreduce_unpack_kernel_dev<T, G, W>), dim3(grid), dim3(kBlock),
+                         reduce_lds(grid, reduce_waves(sizeof(T), W)), stream, slice, p);
     });
   }
 };
@@ -301,8 +303,9 @@ struct ArgWide {
   const PieceBatch& b;
   template <int W>
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
-    hipLaunchKernelGGL((allreduce_wide_kernel<In, T, G, W>), dim3(b.first_block[b.count]), dim3(kBlock), 0,
-                       stream, b, p);
+    const int blocks = b.first_block[b.count];
+    hipLaunchKernelGGL((allreduce_wide_kernel<In, T, G, W>), dim3(blocks), dim3(kBlock),
+                       reduce_lds(blocks, reduce_waves(sizeof(In), W)), stream, b, p);
     return hipGetLastError();
   }
 };
@@ -314,7 +317,8 @@ struct DevWide {
   template <int W>
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
-      hipLaunchKernelGGL((allreduce_wide_kernel_dev<In, T, G, W>), dim3(grid), dim3(kBlock), 0, stream, slice, p);
+      hipLaunchKernelGGL((allreduce_wide_kernel_dev<In, T, G, W>), dim3(grid), dim3(kBlock),
+                         reduce_lds(grid, reduce_waves(sizeof(In), W)), stream, slice, p);
     });
   }
 };
@@ -324,8 +328,9 @@ struct ArgPack {
   const PieceBatch& b;
   template <int W>
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
-    hipLaunchKernelGGL((allreduce_pack_kernel<In, T, W>), dim3(b.first_block[b.count]), dim3(kBlock), 0, stream,
-                       b, p);
+    const int blocks = b.first_block[b.count];
+    hipLaunchKernelGGL((allreduce_pack_kernel<In, T, W>), dim3(blocks), dim3(kBlock),
+                       reduce_lds(blocks, reduce_waves(sizeof(In), W)), stream, b, p);
     return hipGetLastError();
   }
 };
@@ -337,7 +342,8 @@ struct DevPack {
   template <int W>
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
-      hipLaunchKernelGGL((allreduce_pack_kernel_dev<In, T, W>), dim3(grid), dim3(kBlock), 0, stream, slice, p);
+      hipLaunchKernelGGL((allreduce_pack_kernel_dev<In, T, W>), dim3(grid), dim3(kBlock),
+                         reduce_lds(grid, reduce_waves(sizeof(In), W)), stream, slice, p);
     });
   }
 };
@@ -609,24 +615,34 @@ __global__ void __launch_bounds__(kBlock) share_kernel_dev(DevTable t, ReducePar
   share_run<In, Acc, Out, WMAX>(v.piece_run(v.block()), p);
 }
 
+// The share kernels' bound on waves per CU.  Only the fp32 sums into fp32 shards
+// have one (bf16 contributions, W = 8, 1.8 GB: 6291 GB/s without, 6459 at 16
+// waves, 6572 at 12); the kernels of the other types spend their time on
+// arithmetic and lose with fewer waves.
+template <typename Acc, typename Out>
+int share_lds(int blocks) {
+  return sizeof(Acc) == 4 && sizeof(Out) == 4 ? reduce_lds(blocks, 12) : 0;
+}
+
 template <typename In, typename Acc, typename Out, int WMAX>
 hipError_t launch_share_dev_w(const DevTable& t, int blocks, const ReduceParams& p, hipStream_t stream) {
   return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
-    hipLaunchKernelGGL((share_kernel_dev<In, Acc, Out, WMAX>), dim3(grid), dim3(kBlock), 0, stream, slice, p);
+    const int lds = share_lds<Acc, Out>(grid);
+    hipLaunchKernelGGL((share_kernel_dev<In, Acc, Out, WMAX>), dim3(grid), dim3(kBlock), lds, stream, slice, p);
   });
 }
 
 template <typename In, typename Acc, typename Out, int WMAX>
 hipError_t launch_share_w(const PieceBatch& b, const ReduceParams& p, hipStream_t stream) {
+  const int blocks = b.first_block[b.count], lds = share_lds<Acc, Out>(blocks);
   if (b.count == 1) {
-    hipLaunchKernelGGL((share_kernel_one<In, Acc, Out, WMAX>), dim3(b.first_block[1]), dim3(kBlock), 0, stream,
+    hipLaunchKernelGGL((share_kernel_one<In, Acc, Out, WMAX>), dim3(blocks), dim3(kBlock), lds, stream,
                        one_run_of(b), p);
   } else if (b.count <= kFewRuns) {
-    hipLaunchKernelGGL((share_kernel_few<In, Acc, Out, WMAX>), dim3(b.first_block[b.count]), dim3(kBlock), 0,
-                       stream, few_runs_of(b), p);
+    hipLaunchKernelGGL((share_kernel_few<In, Acc, Out, WMAX>), dim3(blocks), dim3(kBlock), lds, stream,
+                       few_runs_of(b), p);
   } else {
-    hipLaunchKernelGGL((share_kernel<In, Acc, Out, WMAX>), dim3(b.first_block[b.count]), dim3(kBlock), 0, stream,
-                       b, p);
+    hipLaunchKernelGGL((share_kernel<In, Acc, Out, WMAX>), dim3(blocks), dim3(kBlock), lds, stream, b, p);
   }
   return hipGetLastError();
 }
