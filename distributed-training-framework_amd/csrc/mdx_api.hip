@@ -192,10 +192,7 @@ int run_copy(const mdx_span* spans, int n_spans, int sdt, int ddt, const CopyPar
 template <typename Flush>
 int push_piece(PieceBatch& b, const Rec& r, Flush&& flush) {
   const int k = b.count;
-  b.own[k] = r.a;
-  b.grad[k] = r.b;
-  b.pos[k] = r.pos;
-  b.numel[k] = r.numel;
+  b.run[k] = {r.a, r.b, r.pos, r.numel};
   b.head[k] = r.head;
   b.first_block[k + 1] = b.first_block[k] + r.blocks;
   b.count = k + 1;
@@ -209,6 +206,7 @@ int run_pieces(const mdx_piece* pieces, void* const* grads, int n_pieces, const 
   memset(&b, 0, sizeof(b));
   auto flush = [&]() -> int {
     if (b.count == 0) return MDX_OK;
+    set_hints(b);
     const int rc = status(launch(b));
     memset(&b, 0, sizeof(b));
     return rc;
@@ -232,14 +230,8 @@ void plan_layout(PlanHeader* h, int count, int64_t blocks) {
   off = align8(off + int64_t(count + 1) * 4);
   h->off_head = off;
   off = align8(off + int64_t(count) * 4);
-  h->off_numel = off;
-  off += int64_t(count) * 8;
-  h->off_a = off;
-  off += int64_t(count) * 8;
-  h->off_b = off;
-  off += int64_t(count) * 8;
-  h->off_pos = off;
-  off += int64_t(count) * 8;
+  h->off_run = off;
+  off += int64_t(count) * int64_t(sizeof(RunRec));
   h->off_hint = off;
   off = align8(off + (hint_groups(blocks) + 1) * 4);
   h->bytes = off;
@@ -270,24 +262,18 @@ int build_plan(PlanHeader proto, Gen&& gen, void* plan, int64_t* plan_bytes) {
   memcpy(base, &h, sizeof(h));
   int32_t* fb = reinterpret_cast<int32_t*>(base + h.off_first_block);
   int32_t* hd = reinterpret_cast<int32_t*>(base + h.off_head);
-  int64_t* nm = reinterpret_cast<int64_t*>(base + h.off_numel);
-  uint64_t* a = reinterpret_cast<uint64_t*>(base + h.off_a);
-  uint64_t* b = reinterpret_cast<uint64_t*>(base + h.off_b);
-  int64_t* ps = reinterpret_cast<int64_t*>(base + h.off_pos);
+  RunRec* rr = reinterpret_cast<RunRec*>(base + h.off_run);
   int k = 0;
   fb[0] = 0;
   rc = gen([&](const Rec& r) -> int {
     hd[k] = r.head;
-    nm[k] = r.numel;
-    a[k] = addr(r.a);
-    b[k] = addr(r.b);
-    ps[k] = r.pos;
+    rr[k] = {r.a, r.b, r.pos, r.numel};
     fb[k + 1] = fb[k] + r.blocks;
     ++k;
     return MDX_OK;
   });
   if (rc != MDX_OK) return rc;
-  // Run hints (find_run_hinted): every run has at least one workgroup, so
+  // Run hints (see kHintBlocks): every run has at least one workgroup, so
   // first_block is strictly increasing and one forward sweep finds them.
   int32_t* hint = reinterpret_cast<int32_t*>(base + h.off_hint);
   const int64_t groups = hint_groups(blocks);
@@ -309,10 +295,7 @@ int plan_view(const void* plan, const void* d_plan, int32_t kind, const PlanHead
   const char* d = static_cast<const char*>(d_plan);
   t->first_block = reinterpret_cast<const int32_t*>(d + h->off_first_block);
   t->head = reinterpret_cast<const int32_t*>(d + h->off_head);
-  t->numel = reinterpret_cast<const int64_t*>(d + h->off_numel);
-  t->a = reinterpret_cast<const uint64_t*>(d + h->off_a);
-  t->b = reinterpret_cast<const uint64_t*>(d + h->off_b);
-  t->pos = reinterpret_cast<const int64_t*>(d + h->off_pos);
+  t->run = reinterpret_cast<const RunRec*>(d + h->off_run);
   t->hint = reinterpret_cast<const int32_t*>(d + h->off_hint);
   t->count = h->count;
   t->base = 0;
@@ -489,6 +472,7 @@ int check_pack_fused(const void* const* replicas, int world, int rank, int dtype
   f->p.out = out;
   f->p.world = world;
   f->p.rank = rank;
+  f->p.own_row = const_cast<void*>(replicas[rank]);
   f->p.pre = scale;
   f->p.inv_scale = 1.0f;
   f->p.found_inf = found_inf;
@@ -646,8 +630,7 @@ bool plan_layout_matches(const PlanHeader* h) {
   PlanHeader ref = *h;
   plan_layout(&ref, h->count, h->blocks);
   return ref.bytes == h->bytes && ref.off_first_block == h->off_first_block && ref.off_head == h->off_head &&
-         ref.off_numel == h->off_numel && ref.off_a == h->off_a && ref.off_b == h->off_b &&
-         ref.off_pos == h->off_pos && ref.off_hint == h->off_hint;
+         ref.off_run == h->off_run && ref.off_hint == h->off_hint;
 }
 
 // The device `stream` runs on, which must be the current one.
@@ -828,6 +811,7 @@ int mdx_allreduce_sum(const void* const* replicas, int world, int dtype, const i
   memset(&b, 0, sizeof(b));
   auto flush = [&]() -> int {
     if (b.count == 0) return MDX_OK;
+    set_hints(b);
     const int r = status(launch(b));
     memset(&b, 0, sizeof(b));
     return r;
@@ -856,6 +840,7 @@ int mdx_allreduce_unpack(const void* const* replicas, int world, int dtype, cons
   memset(&b, 0, sizeof(b));
   auto flush = [&]() -> int {
     if (b.count == 0) return MDX_OK;
+    set_hints(b);
     const int r = status(launch_allreduce(dtype, grad_dtype, true, world, b, f.p, st));
     memset(&b, 0, sizeof(b));
     return r;
@@ -880,6 +865,7 @@ int mdx_allreduce_unpack_wide(const void* const* replicas, int world, int wire_d
   memset(&b, 0, sizeof(b));
   auto flush = [&]() -> int {
     if (b.count == 0) return MDX_OK;
+    set_hints(b);
     const int r = status(launch_allreduce_wide(wire_dtype, grad_dtype, world, b, f.p, st));
     memset(&b, 0, sizeof(b));
     return r;
@@ -903,6 +889,7 @@ int mdx_pack_allreduce_unpack(const void* const* replicas, int world, int rank, 
   memset(&b, 0, sizeof(b));
   auto flush = [&]() -> int {
     if (b.count == 0) return MDX_OK;
+    set_hints(b);
     const int r = status(launch_pack_allreduce(wire_dtype, reduce_dtype, world, b, f.p, st));
     f.p.clear = nullptr;  // the flag clear rides on the first dispatch only
     memset(&b, 0, sizeof(b));
@@ -1102,6 +1089,7 @@ int mdx_pack_allreduce_unpack_planned(const void* plan, const void* d_plan, floa
   p.out = reinterpret_cast<void*>(h->out);
   p.world = h->world;
   p.rank = h->rank;
+  p.own_row = reinterpret_cast<void*>(h->replicas[h->rank]);
   p.pre = h->prescale;
   p.inv_scale = inv_scale;
   p.flags = (h->dtype_a == h->reduce_dtype && h->prescale != 1.0f ? kRedPackScale : 0) |

@@ -76,16 +76,16 @@ __device__ __forceinline__ bf16 from_f32<bf16>(float x) {
 }
 
 // fp32 -> fp16: v_cvt_f16_f32 in the default mode (round to nearest even,
-// fp16 subnormals kept, overflow to +-inf); NaNs are rebuilt as torch does.
+// fp16 subnormals kept, overflow to +-inf).  A NaN becomes sign | 0x7E00 |
+// mantissa >> 13, which is what torch's CPU conversion makes of it (checked
+// over all 2^32 fp32 patterns on the device, signalling NaNs included).  The
+// empty asm keeps the compiler from folding a product and its conversion into one
+// v_fma_mixlo_f16 with an addend of +0, which turns a product of -0 into +0.
 template <>
 __device__ __forceinline__ f16 from_f32<f16>(float x) {
-  const uint32_t u = __float_as_uint(x);
+  asm("" : "+v"(x));
   f16 r;
-  if ((u & 0x7fffffffu) > 0x7f800000u) {
-    r.u = uint16_t(((u >> 16) & 0x8000u) | 0x7e00u | ((u >> 13) & 0x3ffu));
-  } else {
-    r.u = __builtin_bit_cast(uint16_t, _Float16(x));
-  }
+  r.u = __builtin_bit_cast(uint16_t, static_cast<_Float16>(x));
   return r;
 }
 
@@ -223,11 +223,6 @@ __device__ __forceinline__ int find_run_in(const int32_t* first_block, int lo, i
 constexpr int kHintShift = 6;
 constexpr int kHintBlocks = 1 << kHintShift;
 
-__device__ __forceinline__ int find_run_hinted(const int32_t* first_block, const int32_t* hint, int blk) {
-  const int g = blk >> kHintShift;
-  return find_run_in(first_block, hint[g], hint[g + 1] + 1, blk);
-}
-
 // One wave stores 1 into *flag if any of its lanes saw a non-finite value.
 // Must be reached by every lane of the wave.
 __device__ __forceinline__ void flag_nonfinite(bool bad, int32_t* flag) {
@@ -295,15 +290,39 @@ int copy_frag_elems(int src_dtype, int dst_dtype);
 // W-way reductions (all-reduce sum, fused all-reduce + unpack, reduce-scatter share)
 // ----------------------------------------------------------------------------
 
+// One run of a reduction as a workgroup reads it: one 32-byte scalar load.
+struct RunRec {
+  const void* a;  // piece own   (device plans of spans: src)
+  void* b;        // piece grad, the fused unpack's destination   (spans: dst)
+  int64_t pos;
+  int64_t numel;
+};
+
+// `hint` narrows the run lookup as in device plans (see kHintBlocks), with
+// groups of 2^hint_shift workgroups: at most kArgHintGroups of them.
+constexpr int kArgHintGroups = 64;
+
 struct PieceBatch {
-  const void* own[kRunsPerLaunch];
-  int64_t pos[kRunsPerLaunch];
-  int64_t numel[kRunsPerLaunch];
-  void* grad[kRunsPerLaunch];  // fused unpack destination (all-reduce + unpack only)
+  RunRec run[kRunsPerLaunch];
   int32_t head[kRunsPerLaunch];
   int32_t first_block[kRunsPerLaunch + 1];
   int32_t count;
+  int32_t hint_shift;
+  int32_t hint[kArgHintGroups + 1];
 };
+
+// Fills the lookup hints of a complete batch (every run has a workgroup).
+inline void set_hints(PieceBatch& b) {
+  const int blocks = b.first_block[b.count];
+  b.hint_shift = 0;
+  while ((blocks - 1) >> b.hint_shift >= kArgHintGroups) ++b.hint_shift;
+  const int groups = ((blocks - 1) >> b.hint_shift) + 1;
+  for (int g = 0, run = 0; g < groups; ++g) {
+    while (run + 1 < b.count && b.first_block[run + 1] <= g << b.hint_shift) ++run;
+    b.hint[g] = run;
+  }
+  b.hint[groups] = b.count - 1;
+}
 
 enum : int32_t {
   kRedPreMul = 1,      // every contribution * pre, rounded to the reduce dtype
@@ -315,6 +334,7 @@ enum : int32_t {
 
 struct ReduceParams {
   const void* peer[MDX_MAX_WORLD];
+  void* own_row;  // fused pack: peer[rank], the row the pack writes
   void* out;  // may be NULL for the fused unpack (bucket not written)
   int32_t world;
   int32_t rank;
@@ -360,29 +380,44 @@ constexpr int share_unroll(int wmax, int frag_in_bytes) {
 // finds few open rows.  Fewer waves in flight keep the requests of a moment
 // closer together in every stream (workgroups start in grid order), so each
 // dispatch asks for LDS it never touches, as much as leaves room for the number
-// of workgroups below on a CU.  Measured on MI355X, GB/s at 32 / 18 / 16 / 12 /
-// 10 / 8 waves per CU, on the real tables (GPT-2-124M fp32 W = 8, GPT-2-medium
-// bf16 W = 4, four Llama-7B layers bf16 into fp32 W = 8, GPT-2-124M fp16 W = 8):
-//   fp32         6171 / 6243 / 6297 / 6467 / 6470 / 6290
-//   bf16         6346 / 6576 / 6579 / 6103 / 5600 / 4984
-//   bf16 -> fp32 5927 / 6151 / 6234 / 6152 / 5939 / 5303
-//   fp16         6057 / 6094 / 6186 / 6090 / 5556 / --
-// The lower end is where the waves' own instructions are no longer hidden: the
-// 16-bit types need more of them per byte.  (Copies, with one load and one store
-// per lane, lose from 25 waves down and are launched without a bound.)
+// of workgroups below on a CU.  Measured on MI355X, GB/s of the fused pack at
+// 32 / 18 / 16 / 12 / 10 / 9 / 8 waves per CU:
+//   fp32         W = 2  6067 6543 6377 6625 6577 6405 6114
+//                W = 4  5990 6282 6354 6498 6589 6577 6484
+//                W = 8  6369 6231 6310 6547 6624 6626 6681
+//   bf16         W = 2  6291 6532 6563 6406 5876 5527 5094
+//                W = 4  6166 6434 6541 6598 6764 6585 6221
+//                W = 8  6307 6209 6318 6572 6649 6683 6750
+//   bf16 -> fp32 W = 4  6061 6472 6473 6365 6267 6059 5716
+//                W = 8  6062 6285 6365 6573 6574 6352 6122
+//                W = 16 5958 5903 5945 6125 6220 6238 6366
+// on single runs; on real tables GPT-2-124M fp32 W = 8 takes 887 us at 32 waves,
+// 870 at 16, 849 at 12 and 842 at 9, GPT-2-medium bf16 W = 4 785, 758, 759 and
+// 828, four Llama-7B layers bf16 into fp32 W = 8 3280, 3200, 3087 and 3064.
+// The lower end is where the waves' own instructions and start-up are no longer
+// hidden: the fewer loads a wave has, and the more it computes, the more waves
+// it takes.  (Copies, with one load and one store per lane, lose from 25 waves
+// down and are launched without a bound, as is W = 1.)
 constexpr int kCus = 256;
+constexpr int kMaxWavesPerCu = 32;
 constexpr int kLdsBytesPerCu = 160 * 1024;
 constexpr int kLdsGranule = 1280;  // a workgroup's LDS is allocated in these
 // LDS bytes that leave room for `waves` one-wave workgroups on a CU.
-constexpr int lds_for_waves(int waves) { return kLdsBytesPerCu / waves / kLdsGranule * kLdsGranule; }
-constexpr int reduce_waves(int in_size, int world) { return in_size == 4 ? (world <= 4 ? 12 : 10) : 16; }
+constexpr int lds_for_waves(int waves) {
+  return waves >= kMaxWavesPerCu ? 0 : kLdsBytesPerCu / waves / kLdsGranule * kLdsGranule;
+}
+constexpr int reduce_waves(int in_size, int out_size, int world) {
+  if (world == 1) return kMaxWavesPerCu;
+  if (in_size < out_size) return world <= 4 ? 16 : (world <= 6 ? 14 : (world <= 8 ? 10 : 8));
+  return world == 2 ? 14 : (world <= 4 ? 12 : 9);
+}
 // The bound pays once a CU gets several times the workgroups it holds; a short
 // dispatch is over before the queues are full, and its start and end take longer
-// with fewer waves (13.5K workgroups, fp32 W = 4: 17.5 us unbounded, 17.2 at 18
+// with fewer waves (13.5K workgroups, fp32 W = 4: 17.5 us unbounded, 17.0 at 21
 // waves, 17.7 at 12; 7.5K workgroups, a share of 77 MB: 16.4, 16.5 at 16, 17.0 at 12).
 inline int reduce_lds(int blocks, int waves) {
   if (blocks < 32 * kCus) return 0;
-  return lds_for_waves(blocks < 128 * kCus ? max_size(waves, 18) : waves);
+  return lds_for_waves(blocks < 128 * kCus ? max_size(waves, 21) : waves);
 }
 
 // Non-SUM all-reduce (mdx_allreduce_op): runs of the replica layout in the
@@ -428,12 +463,9 @@ hipError_t launch_allreduce_wide(int wire_dtype, int grad_dtype, int world, cons
 
 struct DevTable {
   const int32_t* first_block;  // count + 1 entries
-  const int32_t* hint;         // blocks / kHintBlocks + 2 entries (see find_run_hinted)
+  const int32_t* hint;         // blocks / kHintBlocks + 2 entries (see kHintBlocks)
   const int32_t* head;
-  const int64_t* numel;
-  const uint64_t* a;  // span: src    piece: own
-  const uint64_t* b;  // span: dst    piece: grad
-  const int64_t* pos;  // piece position (pieces only)
+  const RunRec* run;
   int32_t count;
   int32_t base;  // plan workgroup of this dispatch's first workgroup (see launch_plan_slices)
 };
@@ -511,16 +543,41 @@ struct SpanArgView {
   }
 };
 
+// The run of workgroup `blk` from a table with hints for its group: the run that
+// holds the group's first workgroup is read at once with its boundary, and only
+// a workgroup past that boundary looks further.  (A lookup that first settles
+// the run, boundary by boundary, and then reads its fields from a column each
+// keeps a wave waiting for two or three more scalar loads before its first
+// vector load.)
+template <typename Make>
+__device__ __forceinline__ auto run_from_hint(const int32_t* first_block, const int32_t* head, const RunRec* run,
+                                              int lo, int hi, int blk, Make&& make) {
+  int s = lo;
+  int32_t begin = first_block[lo], end = first_block[lo + 1], h = head[lo];
+  RunRec r = run[lo];
+  if (blk >= end) {
+    s = find_run_in(first_block, lo + 1, hi + 1, blk);
+    begin = first_block[s];
+    end = first_block[s + 1];
+    h = head[s];
+    r = run[s];
+  }
+  return make(blk - begin, end - begin, r, h);
+}
+
 struct PieceArgView {
   const PieceBatch& t;
   __device__ __forceinline__ int block() const { return int(blockIdx.x); }
   __device__ __forceinline__ PieceRun piece_run(int blk) const {
     const int32_t end0 = t.first_block[1];
-    const PieceRun r0{blk, end0, t.own[0], t.grad[0], t.pos[0], t.numel[0], t.head[0]};
-    if (blk < end0) return r0;  // first_block[0] == 0
-    const int s = find_run_in(t.first_block, 1, t.count, blk);
-    return {blk - t.first_block[s], t.first_block[s + 1] - t.first_block[s], t.own[s], t.grad[s], t.pos[s],
-            t.numel[s], t.head[s]};
+    const RunRec r0 = t.run[0];
+    const int32_t h0 = t.head[0];
+    if (blk < end0) return {blk, end0, r0.a, r0.b, r0.pos, r0.numel, h0};  // first_block[0] == 0
+    const int g = blk >> t.hint_shift;
+    return run_from_hint(t.first_block, t.head, t.run, t.hint[g], t.hint[g + 1], blk,
+                         [](int c, int nblk, const RunRec& r, int32_t h) {
+                           return PieceRun{c, nblk, r.a, r.b, r.pos, r.numel, h};
+                         });
   }
 };
 
@@ -552,7 +609,7 @@ inline SpanOne one_run_of(const SpanBatch& b) {
 }
 
 inline PieceOne one_run_of(const PieceBatch& b) {
-  return {b.own[0], b.grad[0], b.pos[0], b.numel[0], b.head[0], b.first_block[1]};
+  return {b.run[0].a, b.run[0].b, b.run[0].pos, b.run[0].numel, b.head[0], b.first_block[1]};
 }
 
 // Few-piece tables: up to kFewRuns pieces (an FSDP shard that spans a few
@@ -574,10 +631,10 @@ inline PieceFew few_runs_of(const PieceBatch& b) {
   PieceFew f{};
   for (int k = 0; k < kFewRuns; ++k) {
     const bool used = k < b.count;
-    f.own[k] = used ? b.own[k] : nullptr;
-    f.grad[k] = used ? b.grad[k] : nullptr;
-    f.pos[k] = used ? b.pos[k] : 0;
-    f.numel[k] = used ? b.numel[k] : 0;
+    f.own[k] = used ? b.run[k].a : nullptr;
+    f.grad[k] = used ? b.run[k].b : nullptr;
+    f.pos[k] = used ? b.run[k].pos : 0;
+    f.numel[k] = used ? b.run[k].numel : 0;
     f.head[k] = used ? b.head[k] : -1;
   }
   for (int k = 0; k <= kFewRuns; ++k) f.first_block[k] = k <= b.count ? b.first_block[k] : INT32_MAX;
@@ -622,20 +679,24 @@ struct PieceOneView {
   }
 };
 
-// A device plan's a / b columns hold the span's src / dst or the piece's
-// own / grad pointers.
+// A device plan's records hold the span's src / dst or the piece's own / grad
+// pointers.
 struct DevView {
   DevTable t;
   __device__ __forceinline__ int block() const { return t.base + int(blockIdx.x); }
   __device__ __forceinline__ SpanRun span_run(int blk) const {
-    const int s = find_run_hinted(t.first_block, t.hint, blk);
-    return {blk - t.first_block[s], t.first_block[s + 1] - t.first_block[s], reinterpret_cast<const void*>(t.a[s]),
-            reinterpret_cast<void*>(t.b[s]), t.numel[s], t.head[s]};
+    const int g = blk >> kHintShift;
+    return run_from_hint(t.first_block, t.head, t.run, t.hint[g], t.hint[g + 1], blk,
+                         [](int c, int nblk, const RunRec& r, int32_t h) {
+                           return SpanRun{c, nblk, r.a, r.b, r.numel, h};
+                         });
   }
   __device__ __forceinline__ PieceRun piece_run(int blk) const {
-    const int s = find_run_hinted(t.first_block, t.hint, blk);
-    return {blk - t.first_block[s], t.first_block[s + 1] - t.first_block[s], reinterpret_cast<const void*>(t.a[s]),
-            reinterpret_cast<void*>(t.b[s]), t.pos[s], t.numel[s], t.head[s]};
+    const int g = blk >> kHintShift;
+    return run_from_hint(t.first_block, t.head, t.run, t.hint[g], t.hint[g + 1], blk,
+                         [](int c, int nblk, const RunRec& r, int32_t h) {
+                           return PieceRun{c, nblk, r.a, r.b, r.pos, r.numel, h};
+                         });
   }
 };
 
@@ -661,7 +722,8 @@ struct PlanHeader {
   int32_t pad;
   uint64_t replicas[MDX_MAX_WORLD];
   uint64_t out;
-  int64_t off_first_block, off_head, off_numel, off_a, off_b, off_pos;
+  int64_t off_first_block, off_head, off_run;
+  int64_t unused[3];
   int64_t bytes;
   int64_t off_hint;
 };

@@ -46,10 +46,169 @@
 // all-reduce at W = 8).
 #pragma once
 
+#include <type_traits>
+
 #include "mdx_internal.h"
 
 namespace mdx {
 namespace reduce_impl {
+
+// ---------------------------------------------------------------------------
+// Fragment arithmetic
+// ---------------------------------------------------------------------------
+
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// Element `i` of a run, as a scalar base plus a 32-bit byte offset (a run holds
+// at most kMaxRunElems elements): no 64-bit vector arithmetic per stream.
+static_assert(kMaxRunElems * 4 <= int64_t(UINT32_MAX), "a run's byte offsets fit 32 bits");
+template <typename T>
+__device__ __forceinline__ T* at(T* base, uint32_t i) {
+  using Byte = std::conditional_t<std::is_const_v<T>, const char, char>;
+  return reinterpret_cast<T*>(reinterpret_cast<Byte*>(base) + i * uint32_t(sizeof(T)));
+}
+
+// Two fp32 values rounded to T, the low half first; NaNs as from_f32<T> stores
+// them (bf16: 0xFFFF; `kRaw` leaves the instruction's own quiet NaN, which a
+// following from_f32 or RankSum::get makes 0xFFFF).
+template <typename T, bool kRaw = false>
+__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+  if constexpr (std::is_same_v<T, bf16>) {
+    uint32_t w = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
+    if constexpr (!kRaw) {
+      w = __builtin_isnan(lo) ? w | 0xffffu : w;
+      w = __builtin_isnan(hi) ? w | 0xffff0000u : w;
+    }
+    return w;
+  } else {
+    asm("" : "+v"(lo), "+v"(hi));  // as in from_f32<f16>
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, f16x2));
+  }
+}
+
+// The rank-ordered sum of E elements of T, one rounding to T per add: `first`
+// takes rank 0's values, `add` the next rank's, `get` gives the sums.  The
+// results are those of acc = from_f32<T>(to_f32(acc) + to_f32(x)), bit for bit.
+template <typename T, int E>
+struct RankSum;
+
+template <int E>
+struct RankSum<float, E> {
+  float a[E];
+  __device__ __forceinline__ void first(const float (&x)[E]) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) a[k] = x[k];
+  }
+  __device__ __forceinline__ void add(const float (&x)[E]) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) a[k] += x[k];
+  }
+  __device__ __forceinline__ void get(float (&y)[E]) const {
+#pragma unroll
+    for (int k = 0; k < E; ++k) y[k] = a[k];
+  }
+};
+
+// bf16: the running sum is kept as the fp32 value of its rounding, two elements
+// per v_cvt_pk_bf16_f32, and the NaN encoding is settled once, in `get` (a NaN
+// stays a NaN through the adds): 3.5 instructions per element and add instead
+// of 6 with a conversion, compare and select of its own for each.
+template <int E>
+struct RankSum<bf16, E> {
+  float a[E];
+  __device__ __forceinline__ void first(const bf16 (&x)[E]) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) a[k] = to_f32(x[k]);
+  }
+  __device__ __forceinline__ void add(const bf16 (&x)[E]) {
+#pragma unroll
+    for (int k = 0; k < E; k += 2) {
+      const uint32_t w = pack2<bf16, true>(a[k] + to_f32(x[k]), a[k + 1] + to_f32(x[k + 1]));
+      a[k] = __uint_as_float(w << 16);
+      a[k + 1] = __uint_as_float(w & 0xffff0000u);
+    }
+  }
+  __device__ __forceinline__ void get(bf16 (&y)[E]) const {
+#pragma unroll
+    for (int k = 0; k < E; k += 2) {
+      uint32_t w = (__float_as_uint(a[k]) >> 16) | (__float_as_uint(a[k + 1]) & 0xffff0000u);
+      w = __builtin_isnan(a[k]) ? w | 0xffffu : w;
+      w = __builtin_isnan(a[k + 1]) ? w | 0xffff0000u : w;
+      __builtin_memcpy(&y[k], &w, 4);
+    }
+  }
+};
+
+// fp16: v_pk_add_f16, two elements per instruction.  One fp16 rounding of the
+// exact sum is the fp32 sum rounded to fp16 (an fp32 significand holds 2 * 11 +
+// 2 bits, so rounding twice is rounding once), as over all 2^32 pairs of
+// patterns on the device (of two NaNs, either may be the one that stays).
+template <int E>
+struct RankSum<f16, E> {
+  f16x2 a[E / 2];
+  __device__ __forceinline__ void first(const f16 (&x)[E]) { __builtin_memcpy(a, x, sizeof(a)); }
+  __device__ __forceinline__ void add(const f16 (&x)[E]) {
+    f16x2 b[E / 2];
+    __builtin_memcpy(b, x, sizeof(b));
+#pragma unroll
+    for (int k = 0; k < E / 2; ++k) a[k] = a[k] + b[k];
+  }
+  __device__ __forceinline__ void get(f16 (&y)[E]) const { __builtin_memcpy(y, a, sizeof(a)); }
+};
+
+// A fragment multiplied by `s`, each product rounded to T.
+template <typename T, int E>
+__device__ __forceinline__ void scale_fragment(T (&x)[E], float s) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) x[k] = x[k] * s;
+  } else {
+#pragma unroll
+    for (int k = 0; k < E; k += 2) {
+      const uint32_t w = pack2<T>(to_f32(x[k]) * s, to_f32(x[k + 1]) * s);
+      __builtin_memcpy(&x[k], &w, 4);
+    }
+  }
+}
+
+template <typename S, typename D, int E>
+__device__ __forceinline__ void convert_fragment(const S (&x)[E], D (&y)[E]) {
+  if constexpr (std::is_same_v<S, D> || sizeof(D) == 4) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) y[k] = Cvt<S, D>::run(x[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < E; k += 2) {
+      const uint32_t w = pack2<D>(to_f32(x[k]), to_f32(x[k + 1]));
+      __builtin_memcpy(&y[k], &w, 4);
+    }
+  }
+}
+
+// Whether any element of the fragment is an inf or a NaN.
+template <typename T, int E>
+__device__ __forceinline__ bool any_nonfinite(const T (&x)[E]) {
+  if constexpr (sizeof(T) == 4) {
+    bool bad = false;
+#pragma unroll
+    for (int k = 0; k < E; ++k) bad |= !is_finite(x[k]);
+    return bad;
+  } else {
+    // an all-ones exponent leaves a zero half in the complement
+    constexpr uint32_t kExp = std::is_same_v<T, bf16> ? 0x7f807f80u : 0x7c007c00u;
+    u16x2 least{0xffff, 0xffff};
+#pragma unroll
+    for (int k = 0; k < E; k += 2) {
+      uint32_t w;
+      __builtin_memcpy(&w, &x[k], 4);
+      least = __builtin_elementwise_min(least, __builtin_bit_cast(u16x2, ~w & kExp));
+    }
+    return least.x == 0 || least.y == 0;
+  }
+}
 
 // ---------------------------------------------------------------------------
 // all-reduce (+ fused unpack)
@@ -76,8 +235,10 @@ __device__ __forceinline__ void allreduce_body(const View& tab, const ReducePara
   const int c = run.c;
   const int nblk = run.nblk;
   const int64_t pos = run.pos;
-  const int64_t n = run.numel;
-  const int32_t h = run.head;
+  // A run holds at most kMaxRunElems elements, so its element indices and byte
+  // offsets fit 32 bits: every access is a scalar base plus a 32-bit offset.
+  const int n = int(run.numel);
+  const int h = run.head;
   const int rank = p.rank;
   const int t = int(threadIdx.x);
   const bool unscale = (p.flags & kRedUnscale) != 0;
@@ -85,14 +246,14 @@ __device__ __forceinline__ void allreduce_body(const View& tab, const ReducePara
   const float pre = p.pre;
 
   // Replica `rank` is read through the run's own pointer: the rank's packed
-  // row, or with PACK its gradient (NULL = zeros), packed here.
+  // row, or with PACK its gradient, packed here.  A NULL gradient counts as
+  // zeros; the row it is packed into is read in its place and not used.
+  const bool own_zero = PACK && run.own == nullptr;
+  In* own_row = PACK ? static_cast<In*>(const_cast<void*>(p.own_row)) + pos : nullptr;
+  const In* own = own_zero ? own_row : static_cast<const In*>(run.own);
   const In* src[W];
 #pragma unroll
-  for (int r = 0; r < W; ++r) {
-    src[r] = (r == rank) ? static_cast<const In*>(run.own) : static_cast<const In*>(p.peer[r]) + pos;
-  }
-  const bool own_zero = PACK && run.own == nullptr;
-  In* own_row = PACK ? static_cast<In*>(const_cast<void*>(p.peer[rank])) + pos : nullptr;
+  for (int r = 0; r < W; ++r) src[r] = (r == rank) ? own : static_cast<const In*>(p.peer[r]) + pos;
   const bool pack_scale = PACK && !PRE && (p.flags & kRedPackScale) != 0;
   T* out = p.out ? static_cast<T*>(p.out) + pos : nullptr;
   G* grad = static_cast<G*>(run.grad);
@@ -124,17 +285,15 @@ __device__ __forceinline__ void allreduce_body(const View& tab, const ReducePara
     bad |= !is_finite(g);
     return g;
   };
-  auto element = [&](int64_t i) {
+  auto element = [&](int i) {
     T acc = zero_of<T>();
     In packed = zero_of<In>();
 #pragma unroll
     for (int r = 0; r < W; ++r) {
-      In xr;
+      In xr = src[r][i];
       if (PACK && r == rank) {
-        xr = pack_op(own_zero ? zero_of<In>() : src[r][i]);
+        xr = pack_op(own_zero ? zero_of<In>() : xr);
         packed = xr;
-      } else {
-        xr = src[r][i];
       }
       const T a = widen(xr);
       acc = (r == 0) ? a : from_f32<T>(to_f32(acc) + to_f32(a));
@@ -145,11 +304,11 @@ __device__ __forceinline__ void allreduce_body(const View& tab, const ReducePara
   };
 
   if (h >= 0) {
-    const int64_t nvec = (n - h) / E;
+    const int nvec = (n - h) / E;
     In x[U][W][E];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t v = int64_t(c) * VPB + int64_t(u) * kBlock + t;
+      const int v = c * VPB + u * kBlock + t;
       if constexpr (kWave) {
 #pragma unroll
         for (int r = 0; r < W; ++r) {
@@ -159,77 +318,85 @@ __device__ __forceinline__ void allreduce_body(const View& tab, const ReducePara
       }
       if (v < nvec) {
 #pragma unroll
-        for (int r = 0; r < W; ++r) {
-          if (PACK && r == rank && own_zero) {
-#pragma unroll
-            for (int e = 0; e < E; ++e) x[u][r][e] = zero_of<In>();
-          } else {
-            vload<In, E, true>(x[u][r], src[r] + h + v * E);
-          }
-        }
+        for (int r = 0; r < W; ++r) vload<In, E, true>(x[u][r], at(src[r], uint32_t(h + v * E)));
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t v0 = int64_t(c) * VPB + int64_t(u) * kBlock;  // the fragment of lane 0
-      const int64_t v = v0 + t;
+      const int v0 = c * VPB + u * kBlock;  // the fragment of lane 0
+      const int v = v0 + t;
       const bool active = v < nvec;
       // elements of this wave's fragment that exist (wave-permuted stores only)
-      const int limit = int(max_size(0, int(min_i64(nvec - v0, kBlock)))) * E;
+      const int limit = max_size(0, min_size(nvec - v0, kBlock)) * E;
       if (kWave || active) {
-        const int64_t i = h + v * E;
+        const uint32_t i = uint32_t(h + v * E);
         if constexpr (PACK) {
           // This rank's fragment, packed in registers (static indices: the
           // branch on the wave-uniform rank picks the replica slot).
           In po[E];
 #pragma unroll
-          for (int e = 0; e < E; ++e) po[e] = zero_of<In>();
-#pragma unroll
           for (int r = 0; r < W; ++r) {
             if (r == rank) {
+              __builtin_amdgcn_sched_barrier(0);  // keeps the branch: as selects this runs for every r
+              if (own_zero) {
 #pragma unroll
-              for (int e = 0; e < E; ++e) {
-                x[u][r][e] = pack_op(x[u][r][e]);
-                po[e] = x[u][r][e];
+                for (int e = 0; e < E; ++e) x[u][r][e] = zero_of<In>();
               }
+              if constexpr (!PRE) {
+                if (pack_scale) scale_fragment(x[u][r], pre);
+              }
+#pragma unroll
+              for (int e = 0; e < E; ++e) po[e] = x[u][r][e];
             }
           }
-          if (active) vstore<In, E, true>(own_row + i, po);
+          if (active) vstore<In, E, true>(at(own_row, i), po);
         }
         T y[E];
+        if constexpr (PRE) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-          T acc = widen(x[u][0][e]);
+          for (int e = 0; e < E; ++e) {
+            T acc = widen(x[u][0][e]);
 #pragma unroll
-          for (int r = 1; r < W; ++r) acc = from_f32<T>(to_f32(acc) + to_f32(widen(x[u][r][e])));
-          y[e] = acc;
+            for (int r = 1; r < W; ++r) acc = from_f32<T>(to_f32(acc) + to_f32(widen(x[u][r][e])));
+            y[e] = acc;
+          }
+        } else if constexpr (W == 1) {
+#pragma unroll
+          for (int e = 0; e < E; ++e) y[e] = x[u][0][e];
+        } else {
+          RankSum<T, E> sum;
+          sum.first(x[u][0]);
+#pragma unroll
+          for (int r = 1; r < W; ++r) sum.add(x[u][r]);
+          sum.get(y);
         }
         if (out) {
           if constexpr (kWaveT) {
-            vstore_wave8<T>(out + h + v0 * E, y, t, limit);
+            vstore_wave8<T>(out + uint32_t(h + v0 * E), y, t, limit);
           } else if (active) {
-            vstore<T, E, true>(out + i, y);
+            vstore<T, E, true>(at(out, i), y);
           }
         }
         if constexpr (UNPACK) {
           G gy[E];
-#pragma unroll
-          for (int e = 0; e < E; ++e) gy[e] = finish(y[e]);
+          convert_fragment(y, gy);
+          if (unscale) scale_fragment(gy, inv);
+          bad |= any_nonfinite(gy);
           if constexpr (kWaveG) {
-            vstore_wave8<G>(grad + h + v0 * E, gy, t, limit);
+            vstore_wave8<G>(grad + uint32_t(h + v0 * E), gy, t, limit);
           } else if (active) {
-            vstore<G, E, true>(grad + i, gy);
+            vstore<G, E, true>(at(grad, i), gy);
           }
         }
       }
     }
     if (c == 0 && t < h && t < n) element(t);
-    const int64_t tail0 = h + nvec * E;
+    const int tail0 = h + nvec * E;
     if (c == nblk - 1 && tail0 + t < n) element(tail0 + t);
   } else {
 #pragma unroll 4
     for (int k = 0; k < U * E; ++k) {
-      const int64_t i = int64_t(c) * EPB + int64_t(k) * kBlock + t;
+      const int i = c * EPB + k * kBlock + t;
       if (i < n) element(i);
     }
   }
@@ -280,7 +447,7 @@ struct ArgAllreduce {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     const int blocks = b.first_block[b.count];
     hipLaunchKernelGGL((allreduce_kernel<T, G, W, UNPACK>), dim3(blocks), dim3(kBlock),
-                       reduce_lds(blocks, reduce_waves(sizeof(T), W)), stream, b, p);
+                       reduce_lds(blocks, reduce_waves(sizeof(T), sizeof(T), W)), stream, b, p);
     return hipGetLastError();
   }
 };
@@ -293,7 +460,7 @@ struct DevAllreduceUnpack {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
       hipLaunchKernelGGL((allreduce_unpack_kernel_dev<T, G, W>), dim3(grid), dim3(kBlock),
-                         reduce_lds(grid, reduce_waves(sizeof(T), W)), stream, slice, p);
+                         reduce_lds(grid, reduce_waves(sizeof(T), sizeof(T), W)), stream, slice, p);
     });
   }
 };
@@ -305,7 +472,7 @@ struct ArgWide {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     const int blocks = b.first_block[b.count];
     hipLaunchKernelGGL((allreduce_wide_kernel<In, T, G, W>), dim3(blocks), dim3(kBlock),
-                       reduce_lds(blocks, reduce_waves(sizeof(In), W)), stream, b, p);
+                       reduce_lds(blocks, reduce_waves(sizeof(In), sizeof(T), W)), stream, b, p);
     return hipGetLastError();
   }
 };
@@ -318,7 +485,7 @@ struct DevWide {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
       hipLaunchKernelGGL((allreduce_wide_kernel_dev<In, T, G, W>), dim3(grid), dim3(kBlock),
-                         reduce_lds(grid, reduce_waves(sizeof(In), W)), stream, slice, p);
+                         reduce_lds(grid, reduce_waves(sizeof(In), sizeof(T), W)), stream, slice, p);
     });
   }
 };
@@ -330,7 +497,7 @@ struct ArgPack {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     const int blocks = b.first_block[b.count];
     hipLaunchKernelGGL((allreduce_pack_kernel<In, T, W>), dim3(blocks), dim3(kBlock),
-                       reduce_lds(blocks, reduce_waves(sizeof(In), W)), stream, b, p);
+                       reduce_lds(blocks, reduce_waves(sizeof(In), sizeof(T), W)), stream, b, p);
     return hipGetLastError();
   }
 };
@@ -343,7 +510,7 @@ struct DevPack {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
       hipLaunchKernelGGL((allreduce_pack_kernel_dev<In, T, W>), dim3(grid), dim3(kBlock),
-                         reduce_lds(grid, reduce_waves(sizeof(In), W)), stream, slice, p);
+                         reduce_lds(grid, reduce_waves(sizeof(In), sizeof(T), W)), stream, slice, p);
     });
   }
 };

@@ -151,6 +151,25 @@ def test_pack_allreduce_unpack_planned_matches_direct(rng, wdt, bdt, W, rank):
     _check(c, numels, W, rank, wdt, bdt, 2.0**-10, flag)
 
 
+@pytest.mark.parametrize("planned", [False, True])
+@pytest.mark.parametrize("wdt,bdt", [(o.F32, o.F32), (o.BF16, o.BF16), (o.F16, o.F16), (o.BF16, o.F32)])
+def test_pack_allreduce_unpack_run_lookup(rng, planned, wdt, bdt):
+    """One full table (48 runs) in which groups of workgroups start inside a long run and hold many
+    one-workgroup runs behind it: every workgroup finds its run from the group's hint."""
+    numels = [200_003, *[5] * 15, 1, 60_000, *[300] * 12, 2, 257, 90_001, *[64] * 14, 40_000]
+    assert len(numels) == 48
+    c = _case(rng, wdt, bdt, 2, 1, numels)
+    reps = [r.data_ptr() for r in c["reps"]]
+    flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+    if planned:
+        plan = nat.plan_pack_allreduce_unpack(reps, 1, code(wdt), c["runs"], c["out"].data_ptr(), code(bdt), 0.5, DEV)
+        nat.pack_allreduce_unpack_planned(plan, nat.f32(2.0**-3), flag.data_ptr(), None, stream())
+    else:
+        nat.pack_allreduce_unpack(reps, 1, code(wdt), c["runs"], c["out"].data_ptr(), code(bdt), 0.5, nat.f32(2.0**-3),
+                                  flag.data_ptr(), None, stream())
+    _check(c, numels, 2, 1, wdt, bdt, 2.0**-3, flag)
+
+
 def test_pack_allreduce_unpack_run_past_the_run_limit(rng):
     """A gradient longer than one run (2^26 elements) is cut into runs whose offsets line up."""
     n = (1 << 26) + 1000
