@@ -414,10 +414,19 @@ constexpr int reduce_waves(int in_size, int out_size, int world) {
 // The bound pays once a CU gets several times the workgroups it holds; a short
 // dispatch is over before the queues are full, and its start and end take longer
 // with fewer waves (13.5K workgroups, fp32 W = 4: 17.5 us unbounded, 17.0 at 21
-// waves, 17.7 at 12; 7.5K workgroups, a share of 77 MB: 16.4, 16.5 at 16, 17.0 at 12).
-inline int reduce_lds(int blocks, int waves) {
+// waves, 17.6 at 12; 7.5K workgroups, a share of 77 MB: 16.5, 16.5 at 25, 17.1 at
+// 12).  In between, a single bucket's launch (25-32 MB), 12 waves serve every
+// fp32 and same-type case (fp32 W = 8, 25.6K workgroups: 45.3 us unbounded, 46.0 at
+// 21 waves, 44.1 at 12, 43.6 at 10); a widening one keeps 14, because rows a power
+// of two apart, as square layers of 4096 make them, answer later (33.6 MB buckets
+// launched from backward's hooks, W = 8, whole step: 1178 us unbounded, 1161 at
+// 16, 1162 at 14, 1170 at 12, 1189 at 10).
+inline int reduce_lds(int blocks, int in_size, int out_size, int world) {
+  int waves = reduce_waves(in_size, out_size, world);
   if (blocks < 32 * kCus) return 0;
-  return lds_for_waves(blocks < 128 * kCus ? max_size(waves, 21) : waves);
+  if (blocks < 64 * kCus) waves = max_size(waves, 21);
+  else if (blocks < 256 * kCus) waves = max_size(waves, in_size < out_size ? 14 : 12);
+  return lds_for_waves(waves);
 }
 
 // Non-SUM all-reduce (mdx_allreduce_op): runs of the replica layout in the

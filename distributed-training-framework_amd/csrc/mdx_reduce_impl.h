@@ -447,7 +447,7 @@ struct ArgAllreduce {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     const int blocks = b.first_block[b.count];
     hipLaunchKernelGGL((allreduce_kernel<T, G, W, UNPACK>), dim3(blocks), dim3(kBlock),
-                       reduce_lds(blocks, reduce_waves(sizeof(T), sizeof(T), W)), stream, b, p);
+                       reduce_lds(blocks, sizeof(T), sizeof(T), W), stream, b, p);
     return hipGetLastError();
   }
 };
@@ -460,7 +460,7 @@ struct DevAllreduceUnpack {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
       hipLaunchKernelGGL((allreduce_unpack_kernel_dev<T, G, W>), dim3(grid), dim3(kBlock),
-                         reduce_lds(grid, reduce_waves(sizeof(T), sizeof(T), W)), stream, slice, p);
+                         reduce_lds(grid, sizeof(T), sizeof(T), W), stream, slice, p);
     });
   }
 };
@@ -472,7 +472,7 @@ struct ArgWide {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     const int blocks = b.first_block[b.count];
     hipLaunchKernelGGL((allreduce_wide_kernel<In, T, G, W>), dim3(blocks), dim3(kBlock),
-                       reduce_lds(blocks, reduce_waves(sizeof(In), sizeof(T), W)), stream, b, p);
+                       reduce_lds(blocks, sizeof(In), sizeof(T), W), stream, b, p);
     return hipGetLastError();
   }
 };
@@ -485,7 +485,7 @@ struct DevWide {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
       hipLaunchKernelGGL((allreduce_wide_kernel_dev<In, T, G, W>), dim3(grid), dim3(kBlock),
-                         reduce_lds(grid, reduce_waves(sizeof(In), sizeof(T), W)), stream, slice, p);
+                         reduce_lds(grid, sizeof(In), sizeof(T), W), stream, slice, p);
     });
   }
 };
@@ -497,7 +497,7 @@ struct ArgPack {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     const int blocks = b.first_block[b.count];
     hipLaunchKernelGGL((allreduce_pack_kernel<In, T, W>), dim3(blocks), dim3(kBlock),
-                       reduce_lds(blocks, reduce_waves(sizeof(In), sizeof(T), W)), stream, b, p);
+                       reduce_lds(blocks, sizeof(In), sizeof(T), W), stream, b, p);
     return hipGetLastError();
   }
 };
@@ -510,7 +510,7 @@ struct DevPack {
   hipError_t go(const ReduceParams& p, hipStream_t stream) const {
     return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
       hipLaunchKernelGGL((allreduce_pack_kernel_dev<In, T, W>), dim3(grid), dim3(kBlock),
-                         reduce_lds(grid, reduce_waves(sizeof(In), sizeof(T), W)), stream, slice, p);
+                         reduce_lds(grid, sizeof(In), sizeof(T), W), stream, slice, p);
     });
   }
 };
@@ -783,12 +783,13 @@ __global__ void __launch_bounds__(kBlock) share_kernel_dev(DevTable t, ReducePar
 }
 
 // The share kernels' bound on waves per CU.  Only the fp32 sums into fp32 shards
-// have one (bf16 contributions, W = 8, 1.8 GB: 6291 GB/s without, 6459 at 16
-// waves, 6572 at 12); the kernels of the other types spend their time on
-// arithmetic and lose with fewer waves.
+// have one (bf16 contributions, W = 8, GB/s at 32 / 16 / 12 / 9 waves: 1.8 GB 6239
+// 6431 6547 6558, 288 MB 5761 5916 6215 6266, 144 MB 5535 5514 5510 5481); the kernels
+// of the other types spend their time on arithmetic and lose with fewer waves.
 template <typename Acc, typename Out>
 int share_lds(int blocks) {
-  return sizeof(Acc) == 4 && sizeof(Out) == 4 ? reduce_lds(blocks, 12) : 0;
+  if (sizeof(Acc) != 4 || sizeof(Out) != 4 || blocks < 64 * kCus) return 0;
+  return lds_for_waves(12);
 }
 
 template <typename In, typename Acc, typename Out, int WMAX>
