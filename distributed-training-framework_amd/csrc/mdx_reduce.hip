@@ -33,11 +33,11 @@ hipError_t launch_pack_allreduce_dev_wide(int wire_dtype, int world, const DevTa
                                           const ReduceParams& p, hipStream_t stream);
 hipError_t launch_share_fast(int in_dtype, int wmax, const PieceBatch& b, const ReduceParams& p,
                              hipStream_t stream);
-hipError_t launch_share_generic_f32(int acc_dtype, int out_dtype, const PieceBatch& b, const ReduceParams& p,
+hipError_t launch_share_generic_f32(int acc_dtype, int out_dtype, int wmax, const PieceBatch& b, const ReduceParams& p,
                                     hipStream_t stream);
-hipError_t launch_share_generic_bf16(int acc_dtype, int out_dtype, const PieceBatch& b, const ReduceParams& p,
+hipError_t launch_share_generic_bf16(int acc_dtype, int out_dtype, int wmax, const PieceBatch& b, const ReduceParams& p,
                                      hipStream_t stream);
-hipError_t launch_share_generic_f16(int acc_dtype, int out_dtype, const PieceBatch& b, const ReduceParams& p,
+hipError_t launch_share_generic_f16(int acc_dtype, int out_dtype, int wmax, const PieceBatch& b, const ReduceParams& p,
                                     hipStream_t stream);
 
 hipError_t launch_allreduce(int dtype, int grad_dtype, bool unpack, int world, const PieceBatch& b,
@@ -83,16 +83,16 @@ static bool fast_triple(int in_dtype, int acc_dtype, int out_dtype) {
 }
 
 int share_wmax(int in_dtype, int acc_dtype, int out_dtype, int world) {
-  if (!fast_triple(in_dtype, acc_dtype, out_dtype)) return 16;
+  if (!fast_triple(in_dtype, acc_dtype, out_dtype)) return world <= 4 ? 4 : (world <= 8 ? 8 : 16);
   return world <= 2 ? 2 : (world <= 4 ? 4 : (world <= 8 ? 8 : 16));
 }
 
 hipError_t launch_share(int in_dtype, int acc_dtype, int out_dtype, int wmax, const PieceBatch& b,
                         const ReduceParams& p, hipStream_t stream) {
   if (fast_triple(in_dtype, acc_dtype, out_dtype)) return launch_share_fast(in_dtype, wmax, b, p, stream);
-  if (in_dtype == MDX_BF16) return launch_share_generic_bf16(acc_dtype, out_dtype, b, p, stream);
-  if (in_dtype == MDX_F16) return launch_share_generic_f16(acc_dtype, out_dtype, b, p, stream);
-  return launch_share_generic_f32(acc_dtype, out_dtype, b, p, stream);
+  if (in_dtype == MDX_BF16) return launch_share_generic_bf16(acc_dtype, out_dtype, wmax, b, p, stream);
+  if (in_dtype == MDX_F16) return launch_share_generic_f16(acc_dtype, out_dtype, wmax, b, p, stream);
+  return launch_share_generic_f32(acc_dtype, out_dtype, wmax, b, p, stream);
 }
 
 }  // namespace mdx

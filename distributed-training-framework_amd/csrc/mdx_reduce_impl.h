@@ -34,8 +34,8 @@
 // share_kernel<In, Acc, Out, WMAX>: FSDP's reduce-scatter share, runtime
 // W <= WMAX.  x_r = cvt_Acc(contribution_r[p]); x_r = rnd_Acc(x_r * pre | x_r / pre);
 // acc = rank-ordered sum in Acc; y = cvt_Out(acc); y = rnd_Out(out + y) when
-// accumulating; optional unscale + found-inf epilogue.  The pre-scale and the
-// accumulate are compile-time variants selected once per workgroup.  A piece
+// accumulating; optional unscale + found-inf epilogue.  The pre-scale is a
+// compile-time variant selected once per workgroup.  A piece
 // may carry its own destination (PieceRun::grad), so that one dispatch writes
 // the shard gradients of several FSDP units (the multi-unit share); otherwise
 // it writes out + its position.
@@ -613,7 +613,22 @@ hipError_t launch_pack_dev_for(int world, const DevTable& t, int blocks, const R
 
 enum : int { kPreNone = 0, kPreMul = 1, kPreDiv = 2 };
 
-template <typename In, typename Acc, typename Out, int WMAX, int PRE, bool ACC>
+// A fragment divided by `s`, each quotient rounded to T.
+template <typename T, int E>
+__device__ __forceinline__ void divide_fragment(T (&x)[E], float s) {
+  if constexpr (sizeof(T) == 4) {
+#pragma unroll
+    for (int k = 0; k < E; ++k) x[k] = x[k] / s;
+  } else {
+#pragma unroll
+    for (int k = 0; k < E; k += 2) {
+      const uint32_t w = pack2<T>(to_f32(x[k]) / s, to_f32(x[k + 1]) / s);
+      __builtin_memcpy(&x[k], &w, 4);
+    }
+  }
+}
+
+template <typename In, typename Acc, typename Out, int WMAX, int PRE>
 __device__ __forceinline__ void share_body(const PieceRun& run, const ReduceParams& p) {
   constexpr int E = reduce_frag_elems(int(sizeof(In)), int(sizeof(Out)), int(sizeof(Out)));
   constexpr int U = share_unroll(WMAX, E * int(sizeof(In)));
@@ -627,13 +642,14 @@ __device__ __forceinline__ void share_body(const PieceRun& run, const ReducePara
   const int c = run.c;
   const int nblk = run.nblk;
   const int64_t pos = run.pos;
-  const int64_t n = run.numel;
-  const int32_t h = run.head;
+  const int n = int(run.numel);  // at most kMaxRunElems
+  const int h = run.head;
   const int world = p.world;
   const int rank = p.rank;
   const bool own_zero = (run.own == nullptr);
   const int t = int(threadIdx.x);
   const float pre = p.pre;
+  const bool accumulate = (p.flags & kRedAccumulate) != 0;
   const bool unscale = (p.flags & kRedUnscale) != 0;
   const float inv = p.inv_scale;
 
@@ -653,35 +669,29 @@ __device__ __forceinline__ void share_body(const PieceRun& run, const ReducePara
     if constexpr (PRE == kPreDiv) a = from_f32<Acc>(to_f32(a) / pre);
     return a;
   };
-  auto finish = [&](Acc acc, Out prev) -> Out {
-    Out y = Cvt<Acc, Out>::run(acc);
-    if constexpr (ACC) y = from_f32<Out>(to_f32(prev) + to_f32(y));
-    const Out ys = from_f32<Out>(to_f32(y) * inv);
-    y = unscale ? ys : y;
-    bad |= !is_finite(y);
-    return y;
-  };
-  auto element = [&](int64_t i) {
+  auto element = [&](int i) {
     Acc acc = zero_of<Acc>();
-#pragma unroll
-    for (int r = 0; r < WMAX; ++r) {
-      if (r < world) {
-        const In x = (r == rank && own_zero) ? zero_of<In>() : src[r][i];
-        const Acc a = widen(x);
-        acc = (r == 0) ? a : from_f32<Acc>(to_f32(acc) + to_f32(a));
-      }
+    for (int r = 0; r < world; ++r) {
+      const In* row = (r == rank) ? static_cast<const In*>(run.own) : static_cast<const In*>(p.peer[r]) + pos;
+      const In x = (r == rank && own_zero) ? zero_of<In>() : row[i];
+      const Acc a = widen(x);
+      acc = (r == 0) ? a : from_f32<Acc>(to_f32(acc) + to_f32(a));
     }
-    const Out prev = ACC ? out[i] : zero_of<Out>();
-    out[i] = finish(acc, prev);
+    Out y = Cvt<Acc, Out>::run(acc);
+    if (accumulate) y = from_f32<Out>(to_f32(out[i]) + to_f32(y));
+    if (unscale) y = from_f32<Out>(to_f32(y) * inv);
+    bad |= !is_finite(y);
+    out[i] = y;
   };
 
   if (h >= 0) {
-    const int64_t nvec = (n - h) / E;
+    const int nvec = (n - h) / E;
     In x[U][WMAX][E];
     Out prev[U][E];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t v = int64_t(c) * VPB + int64_t(u) * kBlock + t;
+      const int v = c * VPB + u * kBlock + t;
+      const uint32_t i = uint32_t(h + v * E);
       if constexpr (kWave) {
 #pragma unroll
         for (int k = 0; k < E; ++k) {
@@ -691,7 +701,6 @@ __device__ __forceinline__ void share_body(const PieceRun& run, const ReducePara
         }
       }
       if (v < nvec) {
-        const int64_t i = h + v * E;
 #pragma unroll
         for (int r = 0; r < WMAX; ++r) {
           if (r < world) {
@@ -699,44 +708,64 @@ __device__ __forceinline__ void share_body(const PieceRun& run, const ReducePara
 #pragma unroll
               for (int k = 0; k < E; ++k) x[u][r][k] = zero_of<In>();
             } else {
-              vload<In, E, true>(x[u][r], src[r] + i);
+              vload<In, E, true>(x[u][r], at(src[r], i));
             }
           }
         }
-        if constexpr (ACC) vload<Out, E, false>(prev[u], out + i);
+        if (accumulate) vload<Out, E, false>(prev[u], at(out, i));
       }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t v0 = int64_t(c) * VPB + int64_t(u) * kBlock;  // the fragment of lane 0
-      const int64_t v = v0 + t;
+      const int v0 = c * VPB + u * kBlock;  // the fragment of lane 0
+      const int v = v0 + t;
       const bool active = v < nvec;
-      const int limit = int(max_size(0, int(min_i64(nvec - v0, kBlock)))) * E;
+      const int limit = max_size(0, min_size(nvec - v0, kBlock)) * E;
       if (kWave || active) {
-        Out y[E];
+        // rank 0's values, widened, pre-scaled; then every next rank's added
+        RankSum<Acc, E> sum;
+        Acc a[E];
 #pragma unroll
-        for (int k = 0; k < E; ++k) {
-          Acc acc = widen(x[u][0][k]);
-#pragma unroll
-          for (int r = 1; r < WMAX; ++r) {
-            if (r < world) acc = from_f32<Acc>(to_f32(acc) + to_f32(widen(x[u][r][k])));
+        for (int r = 0; r < WMAX; ++r) {
+          if (r < world) {
+            convert_fragment(x[u][r], a);
+            if constexpr (PRE == kPreMul) scale_fragment(a, pre);
+            if constexpr (PRE == kPreDiv) divide_fragment(a, pre);
+            if (r == 0) sum.first(a);
+            else sum.add(a);
           }
-          y[k] = finish(acc, ACC ? prev[u][k] : zero_of<Out>());
         }
+        // (a world of one hands its values on as they are, NaN payloads too)
+        if (world > 1) sum.get(a);
+        Out y[E];
+        convert_fragment(a, y);
+        if (accumulate) {
+          if constexpr (sizeof(Out) == 4) {
+#pragma unroll
+            for (int k = 0; k < E; ++k) y[k] = prev[u][k] + y[k];
+          } else {
+            RankSum<Out, E> total;
+            total.first(prev[u]);
+            total.add(y);
+            total.get(y);
+          }
+        }
+        if (unscale) scale_fragment(y, inv);
+        bad |= any_nonfinite(y);
         if constexpr (kWave) {
-          vstore_wave8<Out>(out + h + v0 * E, y, t, limit);
+          vstore_wave8<Out>(out + uint32_t(h + v0 * E), y, t, limit);
         } else {
-          vstore<Out, E, true>(out + h + v * E, y);
+          vstore<Out, E, true>(at(out, uint32_t(h + v * E)), y);
         }
       }
     }
     if (c == 0 && t < h && t < n) element(t);
-    const int64_t tail0 = h + nvec * E;
+    const int tail0 = h + nvec * E;
     if (c == nblk - 1 && tail0 + t < n) element(tail0 + t);
   } else {
-#pragma unroll 4
+#pragma unroll 1
     for (int k = 0; k < U * E; ++k) {
-      const int64_t i = int64_t(c) * EPB + int64_t(k) * kBlock + t;
+      const int i = c * EPB + k * kBlock + t;
       if (i < n) element(i);
     }
   }
@@ -745,17 +774,9 @@ __device__ __forceinline__ void share_body(const PieceRun& run, const ReducePara
 
 template <typename In, typename Acc, typename Out, int WMAX>
 __device__ __forceinline__ void share_run(const PieceRun& run, const ReduceParams& p) {
-  const bool acc = (p.flags & kRedAccumulate) != 0;
-  if (p.flags & kRedPreMul) {
-    if (acc) share_body<In, Acc, Out, WMAX, kPreMul, true>(run, p);
-    else share_body<In, Acc, Out, WMAX, kPreMul, false>(run, p);
-  } else if (p.flags & kRedPreDiv) {
-    if (acc) share_body<In, Acc, Out, WMAX, kPreDiv, true>(run, p);
-    else share_body<In, Acc, Out, WMAX, kPreDiv, false>(run, p);
-  } else {
-    if (acc) share_body<In, Acc, Out, WMAX, kPreNone, true>(run, p);
-    else share_body<In, Acc, Out, WMAX, kPreNone, false>(run, p);
-  }
+  if (p.flags & kRedPreMul) share_body<In, Acc, Out, WMAX, kPreMul>(run, p);
+  else if (p.flags & kRedPreDiv) share_body<In, Acc, Out, WMAX, kPreDiv>(run, p);
+  else share_body<In, Acc, Out, WMAX, kPreNone>(run, p);
 }
 
 template <typename In, typename Acc, typename Out, int WMAX>
@@ -782,27 +803,40 @@ __global__ void __launch_bounds__(kBlock) share_kernel_dev(DevTable t, ReducePar
   share_run<In, Acc, Out, WMAX>(v.piece_run(v.block()), p);
 }
 
-// The share kernels' bound on waves per CU.  Only the fp32 sums into fp32 shards
-// have one (bf16 contributions, W = 8, GB/s at 32 / 16 / 12 / 9 waves: 1.8 GB 6239
-// 6431 6547 6558, 288 MB 5761 5916 6215 6266, 144 MB 5535 5514 5510 5481); the kernels
-// of the other types spend their time on arithmetic and lose with fewer waves.
+// The share kernels' bound on waves per CU (see reduce_waves), GB/s at 32 / 18 /
+// 12 / 9 waves:
+//   bf16 -> fp32 sums, W = 8, 1.8 GB        6347 6438 6681 6871   (288 MB: 5761 5843 6215 6266)
+//   bf16 -> bf16 sums -> fp32, W = 4, 630 MB  6310 6421 6574 6376
+//   bf16 sums, W = 8, 1.9 GB                6241 6351 6769 5965
+//   bf16 sums, W = 2, 630 MB                6532 6622 5500 4579
+//   fp16 sums, W = 8, 940 MB                6244 6373 6567 6871
+// A division per contribution (W not a power of two) takes more waves: fp32 sums
+// of fp16, W = 6, 5971 6170 6129 5926 with 6376 at 14; bf16 sums, W = 6, lose with any
+// bound.
 template <typename Acc, typename Out>
-int share_lds(int blocks) {
-  if (sizeof(Acc) != 4 || sizeof(Out) != 4 || blocks < 64 * kCus) return 0;
-  return lds_for_waves(12);
+int share_lds(int blocks, const ReduceParams& p) {
+  if (blocks < 64 * kCus) return 0;
+  const bool divides = (p.flags & kRedPreDiv) != 0;
+  if constexpr (std::is_same_v<Acc, bf16>) {
+    if (divides) return 0;
+    return lds_for_waves(p.world <= 2 ? 18 : (p.world <= 8 ? 12 : 10));
+  } else {
+    if (divides) return sizeof(Acc) == 4 ? lds_for_waves(14) : 0;
+    return lds_for_waves(9);
+  }
 }
 
 template <typename In, typename Acc, typename Out, int WMAX>
 hipError_t launch_share_dev_w(const DevTable& t, int blocks, const ReduceParams& p, hipStream_t stream) {
   return launch_plan_slices(t, blocks, [&](const DevTable& slice, int grid) {
-    const int lds = share_lds<Acc, Out>(grid);
+    const int lds = share_lds<Acc, Out>(grid, p);
     hipLaunchKernelGGL((share_kernel_dev<In, Acc, Out, WMAX>), dim3(grid), dim3(kBlock), lds, stream, slice, p);
   });
 }
 
 template <typename In, typename Acc, typename Out, int WMAX>
 hipError_t launch_share_w(const PieceBatch& b, const ReduceParams& p, hipStream_t stream) {
-  const int blocks = b.first_block[b.count], lds = share_lds<Acc, Out>(blocks);
+  const int blocks = b.first_block[b.count], lds = share_lds<Acc, Out>(blocks, p);
   if (b.count == 1) {
     hipLaunchKernelGGL((share_kernel_one<In, Acc, Out, WMAX>), dim3(blocks), dim3(kBlock), lds, stream,
                        one_run_of(b), p);
@@ -815,25 +849,32 @@ hipError_t launch_share_w(const PieceBatch& b, const ReduceParams& p, hipStream_
   return hipGetLastError();
 }
 
-// Every (Acc, Out) pair for contributions of type In at the widest class
-// (runtime W <= 16), except (fp32, fp32), which has width-specialised kernels.
+// Every (Acc, Out) pair for contributions of type In, except (fp32, fp32), at the
+// width classes of share_wmax.
+template <typename In, typename Acc, typename Out>
+hipError_t launch_share_width(int wmax, const PieceBatch& b, const ReduceParams& p, hipStream_t stream) {
+  if (wmax == 4) return launch_share_w<In, Acc, Out, 4>(b, p, stream);
+  if (wmax == 8) return launch_share_w<In, Acc, Out, 8>(b, p, stream);
+  return launch_share_w<In, Acc, Out, 16>(b, p, stream);
+}
+
 template <typename In, typename Acc>
-hipError_t share16_out(int out_dtype, const PieceBatch& b, const ReduceParams& p, hipStream_t stream) {
-  if (out_dtype == MDX_BF16) return launch_share_w<In, Acc, bf16, 16>(b, p, stream);
-  if (out_dtype == MDX_F16) return launch_share_w<In, Acc, f16, 16>(b, p, stream);
+hipError_t launch_share_out(int out_dtype, int wmax, const PieceBatch& b, const ReduceParams& p, hipStream_t stream) {
+  if (out_dtype == MDX_BF16) return launch_share_width<In, Acc, bf16>(wmax, b, p, stream);
+  if (out_dtype == MDX_F16) return launch_share_width<In, Acc, f16>(wmax, b, p, stream);
   if constexpr (sizeof(Acc) == 4) {
-    return hipErrorInvalidValue;  // (fp32, fp32) goes to the width-specialised kernels
+    return hipErrorInvalidValue;  // (fp32, fp32) goes to launch_share_fast
   } else {
-    return launch_share_w<In, Acc, float, 16>(b, p, stream);
+    return launch_share_width<In, Acc, float>(wmax, b, p, stream);
   }
 }
 
 template <typename In>
-hipError_t launch_share_generic_for(int acc_dtype, int out_dtype, const PieceBatch& b, const ReduceParams& p,
-                                    hipStream_t stream) {
-  if (acc_dtype == MDX_F32) return share16_out<In, float>(out_dtype, b, p, stream);
-  if (acc_dtype == MDX_BF16) return share16_out<In, bf16>(out_dtype, b, p, stream);
-  return share16_out<In, f16>(out_dtype, b, p, stream);
+hipError_t launch_share_generic_for(int acc_dtype, int out_dtype, int wmax, const PieceBatch& b,
+                                    const ReduceParams& p, hipStream_t stream) {
+  if (acc_dtype == MDX_F32) return launch_share_out<In, float>(out_dtype, wmax, b, p, stream);
+  if (acc_dtype == MDX_BF16) return launch_share_out<In, bf16>(out_dtype, wmax, b, p, stream);
+  return launch_share_out<In, f16>(out_dtype, wmax, b, p, stream);
 }
 
 }  // namespace reduce_impl

@@ -1,13 +1,13 @@
 // Instantiates the reduce-scatter share of fp32 contributions for the
-// remaining (reduction, shard) dtype pairs, at the widest class (runtime
-// W <= 16).
+// remaining (reduction, shard) dtype pairs, at every width class
+// (runtime W).
 #include "mdx_reduce_impl.h"
 
 namespace mdx {
 
-hipError_t launch_share_generic_f32(int acc_dtype, int out_dtype, const PieceBatch& b, const ReduceParams& p,
+hipError_t launch_share_generic_f32(int acc_dtype, int out_dtype, int wmax, const PieceBatch& b, const ReduceParams& p,
                                     hipStream_t stream) {
-  return reduce_impl::launch_share_generic_for<float>(acc_dtype, out_dtype, b, p, stream);
+  return reduce_impl::launch_share_generic_for<float>(acc_dtype, out_dtype, wmax, b, p, stream);
 }
 
 }  // namespace mdx

@@ -371,6 +371,16 @@ def test_reduce_scatter_share_piece_counts(rng, k, idt):
     _share_case(rng, numels, idt, o.F32, o.F32, 2, 0, k % 2 == 1)
 
 
+@pytest.mark.parametrize("W,rank", [(1, 0), (4, 3), (5, 2), (8, 7), (9, 0), (16, 11)])
+@pytest.mark.parametrize("idt,rdt,sdt", [(o.BF16, o.BF16, o.F32), (o.BF16, o.BF16, o.BF16), (o.F16, o.F16, o.F16),
+                                         (o.F32, o.F16, o.BF16), (o.F16, o.F32, o.F16)])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_reduce_scatter_share_width_classes(rng, idt, rdt, sdt, W, rank, accumulate):
+    """The edges of the width classes (4, 8, 16 ranks) of the shares that are not fp32 into fp32, with
+    chunks of every lane, a partial chunk, a head and a tail; multiplied and divided by W."""
+    _share_case(rng, [4100 * W + 3, 517 * W, 6, 1031 * W + 1], idt, rdt, sdt, W, rank, accumulate)
+
+
 @pytest.mark.parametrize("seed", range(40))
 def test_reduce_scatter_share_fuzz(seed):
     """Seeded random shares: 1-10 parameters of 1-5000 elements, W in [2, 16], any rank, fp32 / bf16 /
