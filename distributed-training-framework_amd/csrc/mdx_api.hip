@@ -159,8 +159,7 @@ int for_each_piece_run(const mdx_piece* pieces, void* const* grads, int n_pieces
 // Kernel-argument batches (direct entry points)
 // ---------------------------------------------------------------------------
 
-int run_copy(const mdx_span* spans, int n_spans, int sdt, int ddt, const CopyParams& params, bool in_place,
-             hipStream_t stream) {
+int run_copy(const mdx_span* spans, int n_spans, int sdt, int ddt, const CopyParams& params, hipStream_t stream) {
   SpanBatch b;
   memset(&b, 0, sizeof(b));
   CopyParams p = params;  // a requested flag clear rides on the first dispatch only
@@ -171,7 +170,7 @@ int run_copy(const mdx_span* spans, int n_spans, int sdt, int ddt, const CopyPar
     memset(&b, 0, sizeof(b));
     return rc;
   };
-  const int rc = for_each_span_run(spans, n_spans, sdt, ddt, in_place, [&](const Rec& r) -> int {
+  const int rc = for_each_span_run(spans, n_spans, sdt, ddt, false, [&](const Rec& r) -> int {
     const int k = b.count;
     b.src[k] = r.a;
     b.dst[k] = r.b;
@@ -185,6 +184,34 @@ int run_copy(const mdx_span* spans, int n_spans, int sdt, int ddt, const CopyPar
   const int frc = flush();
   if (frc != MDX_OK) return frc;
   // nothing was launched: the clear still has to happen, in stream order
+  return p.clear != nullptr ? status(launch_clear_flag(p.clear, stream)) : MDX_OK;
+}
+
+// The in-place form (each span's `dst` alone), with a table of its own.
+int run_in_place(const mdx_span* spans, int n_spans, int dt, const CopyParams& params, hipStream_t stream) {
+  InPlaceBatch b;
+  b.count = 0;
+  b.first_block[0] = 0;
+  CopyParams p = params;  // a requested flag clear rides on the first dispatch only
+  auto flush = [&]() -> int {
+    if (b.count == 0) return MDX_OK;
+    set_hints(b);
+    const int rc = status(launch_unscale(dt, b, p, stream));
+    p.clear = nullptr;
+    b.count = 0;
+    return rc;
+  };
+  const int rc = for_each_span_run(spans, n_spans, dt, dt, true, [&](const Rec& r) -> int {
+    const int k = b.count;
+    b.data[k] = r.b;
+    b.numel_head[k] = uint32_t(r.numel) | uint32_t(r.head + 1) << kNumelBits;
+    b.first_block[k + 1] = b.first_block[k] + r.blocks;
+    b.count = k + 1;
+    return b.count == kInPlaceRunsPerLaunch ? flush() : MDX_OK;
+  });
+  if (rc != MDX_OK) return rc;
+  const int frc = flush();
+  if (frc != MDX_OK) return frc;
   return p.clear != nullptr ? status(launch_clear_flag(p.clear, stream)) : MDX_OK;
 }
 
@@ -682,7 +709,7 @@ int mdx_pack(const mdx_span* spans, int n_spans, int src_dtype, int dst_dtype, f
   int32_t flags = 0;
   if (scale != 1.0f) flags = divide ? kCopyDivide : kCopyScale;
   CopyParams p{scale, flags, nullptr, clear_flag};
-  return run_copy(spans, n_spans, src_dtype, dst_dtype, p, false, static_cast<hipStream_t>(stream));
+  return run_copy(spans, n_spans, src_dtype, dst_dtype, p, static_cast<hipStream_t>(stream));
 }
 
 int mdx_unpack(const mdx_span* spans, int n_spans, int src_dtype, int dst_dtype, float inv_scale,
@@ -692,17 +719,23 @@ int mdx_unpack(const mdx_span* spans, int n_spans, int src_dtype, int dst_dtype,
   if (rc != MDX_OK) return rc;
   CopyParams p{inv_scale, (inv_scale != 1.0f ? kCopyScale : 0) | (found_inf ? kCopyCheck : 0),
                found_inf, nullptr};
-  return run_copy(spans, n_spans, src_dtype, dst_dtype, p, false, static_cast<hipStream_t>(stream));
+  return run_copy(spans, n_spans, src_dtype, dst_dtype, p, static_cast<hipStream_t>(stream));
 }
 
 int mdx_unscale_found_inf(const mdx_span* spans, int n_spans, int dtype, float inv_scale,
                           int32_t* found_inf, void* stream) {
+  return mdx_unscale_found_inf_clear(spans, n_spans, dtype, inv_scale, found_inf, nullptr, stream);
+}
+
+int mdx_unscale_found_inf_clear(const mdx_span* spans, int n_spans, int dtype, float inv_scale, int32_t* found_inf,
+                                int32_t* clear_flag, void* stream) {
   if (!valid_dtype(dtype)) return MDX_EDTYPE;
   int rc = check_spans(spans, n_spans, false);
   if (rc != MDX_OK) return rc;
+  if (clear_flag != nullptr && clear_flag == found_inf) return MDX_EALIAS;
   CopyParams p{inv_scale, (inv_scale != 1.0f ? kCopyScale : 0) | (found_inf ? kCopyCheck : 0),
-               found_inf, nullptr};
-  return run_copy(spans, n_spans, dtype, dtype, p, true, static_cast<hipStream_t>(stream));
+               found_inf, clear_flag};
+  return run_in_place(spans, n_spans, dtype, p, static_cast<hipStream_t>(stream));
 }
 
 int mdx_cast_f32_bf16(const float* src, uint16_t* dst, int64_t numel, void* stream) {
@@ -710,7 +743,7 @@ int mdx_cast_f32_bf16(const float* src, uint16_t* dst, int64_t numel, void* stre
   if (any_overlap(src, numel * 4, dst, numel * 2)) return MDX_EALIAS;
   mdx_span sp{src, dst, numel};
   CopyParams p{1.0f, 0, nullptr, nullptr};
-  return run_copy(&sp, 1, MDX_F32, MDX_BF16, p, false, static_cast<hipStream_t>(stream));
+  return run_copy(&sp, 1, MDX_F32, MDX_BF16, p, static_cast<hipStream_t>(stream));
 }
 
 int mdx_allreduce_op(const void* const* replicas, int world, int dtype, int op, const int64_t* offsets,

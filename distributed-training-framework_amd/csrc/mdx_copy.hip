@@ -143,6 +143,28 @@ __global__ void __launch_bounds__(kBlock) copy_kernel_dev(DevTable t, CopyParams
   copy_body<S, D, SCALE, CHECK>(DevView{t}, p);
 }
 
+// In-place runs in the kernel-argument segment.
+template <typename T, int SCALE, bool CHECK>
+__global__ void __launch_bounds__(kBlock) copy_kernel_in_place(InPlaceBatch b, CopyParams p) {
+  copy_body<T, T, SCALE, CHECK>(InPlaceView{b}, p);
+}
+
+template <typename T>
+hipError_t launch_unscale_t(const InPlaceBatch& b, const CopyParams& p, hipStream_t stream) {
+  const dim3 grid(b.first_block[b.count]), block(kBlock);
+  const bool check = (p.flags & kCopyCheck) != 0, scale = (p.flags & kCopyScale) != 0;
+  if (check && scale) {
+    hipLaunchKernelGGL((copy_kernel_in_place<T, kScaleMul, true>), grid, block, 0, stream, b, p);
+  } else if (check) {
+    hipLaunchKernelGGL((copy_kernel_in_place<T, kScaleNone, true>), grid, block, 0, stream, b, p);
+  } else if (scale) {
+    hipLaunchKernelGGL((copy_kernel_in_place<T, kScaleMul, false>), grid, block, 0, stream, b, p);
+  } else {
+    hipLaunchKernelGGL((copy_kernel_in_place<T, kScaleNone, false>), grid, block, 0, stream, b, p);
+  }
+  return hipGetLastError();
+}
+
 // Either table kind: a kernel-argument SpanBatch (grid from its prefix; one run goes
 // out as a SpanOne) or a DevTable.
 struct ArgLaunch {
@@ -201,6 +223,12 @@ __global__ void __launch_bounds__(kBlock) clear_flag_kernel(int32_t* flag) {
 }
 
 }  // namespace
+
+hipError_t launch_unscale(int dtype, const InPlaceBatch& b, const CopyParams& p, hipStream_t stream) {
+  if (dtype == MDX_F32) return launch_unscale_t<float>(b, p, stream);
+  if (dtype == MDX_BF16) return launch_unscale_t<bf16>(b, p, stream);
+  return launch_unscale_t<f16>(b, p, stream);
+}
 
 hipError_t launch_clear_flag(int32_t* flag, hipStream_t stream) {
   hipLaunchKernelGGL(clear_flag_kernel, dim3(1), dim3(kBlock), 0, stream, flag);

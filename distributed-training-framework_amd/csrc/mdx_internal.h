@@ -223,6 +223,24 @@ __device__ __forceinline__ int find_run_in(const int32_t* first_block, int lo, i
 constexpr int kHintShift = 6;
 constexpr int kHintBlocks = 1 << kHintShift;
 
+// A kernel-argument batch carries hints of the same kind, with groups of
+// 2^hint_shift workgroups: at most kArgHintGroups of them.
+constexpr int kArgHintGroups = 64;
+
+// Fills the lookup hints of a complete batch (every run has a workgroup).
+template <typename Batch>
+void set_hints(Batch& b) {
+  const int blocks = b.first_block[b.count];
+  b.hint_shift = 0;
+  while ((blocks - 1) >> b.hint_shift >= kArgHintGroups) ++b.hint_shift;
+  const int groups = ((blocks - 1) >> b.hint_shift) + 1;
+  for (int g = 0, run = 0; g < groups; ++g) {
+    while (run + 1 < b.count && b.first_block[run + 1] <= g << b.hint_shift) ++run;
+    b.hint[g] = run;
+  }
+  b.hint[groups] = b.count - 1;
+}
+
 // One wave stores 1 into *flag if any of its lanes saw a non-finite value.
 // Must be reached by every lane of the wave.
 __device__ __forceinline__ void flag_nonfinite(bool bad, int32_t* flag) {
@@ -252,6 +270,25 @@ struct CopyParams {
   int32_t* found_inf;
   int32_t* clear;  // set to 0 by the dispatch's first lane (the scaler's per-step flag clear), or NULL
 };
+
+// In-place runs (unscale): source, destination and type are one, so a run is a
+// pointer and a packed length, and one kernel-argument table holds the ~150
+// gradients of a GPT-2 step, which a SpanBatch spreads over four dispatches of
+// which each starts and drains alone (GPT-2-124M fp16, 148 gradients: 4 x 25.2 us
+// against one dispatch of 78).  The table stays below 4 KB of arguments.
+constexpr int kInPlaceRunsPerLaunch = 224;
+
+struct InPlaceBatch {
+  void* data[kInPlaceRunsPerLaunch];
+  uint32_t numel_head[kInPlaceRunsPerLaunch];  // numel, and head + 1 in the upper bits
+  int32_t first_block[kInPlaceRunsPerLaunch + 1];
+  int32_t count;
+  int32_t hint_shift;
+  int32_t hint[kArgHintGroups + 1];
+};
+constexpr int kNumelBits = 27;
+static_assert(kMaxRunElems < (int64_t(1) << kNumelBits), "a run's length fits its field");
+static_assert(sizeof(InPlaceBatch) + sizeof(CopyParams) <= 4096, "one dispatch's kernel arguments");
 
 // Fragments.  In the W-way reductions a fragment is one 16-byte vector of the
 // widest type the kernel stores, so that every store instruction of a wave
@@ -283,6 +320,7 @@ constexpr int kHeadRange = 8;
 
 hipError_t launch_copy(int src_dtype, int dst_dtype, const SpanBatch& b, const CopyParams& p,
                        hipStream_t stream);
+hipError_t launch_unscale(int dtype, const InPlaceBatch& b, const CopyParams& p, hipStream_t stream);
 hipError_t launch_clear_flag(int32_t* flag, hipStream_t stream);
 int copy_frag_elems(int src_dtype, int dst_dtype);
 
@@ -298,10 +336,6 @@ struct RunRec {
   int64_t numel;
 };
 
-// `hint` narrows the run lookup as in device plans (see kHintBlocks), with
-// groups of 2^hint_shift workgroups: at most kArgHintGroups of them.
-constexpr int kArgHintGroups = 64;
-
 struct PieceBatch {
   RunRec run[kRunsPerLaunch];
   int32_t head[kRunsPerLaunch];
@@ -310,19 +344,6 @@ struct PieceBatch {
   int32_t hint_shift;
   int32_t hint[kArgHintGroups + 1];
 };
-
-// Fills the lookup hints of a complete batch (every run has a workgroup).
-inline void set_hints(PieceBatch& b) {
-  const int blocks = b.first_block[b.count];
-  b.hint_shift = 0;
-  while ((blocks - 1) >> b.hint_shift >= kArgHintGroups) ++b.hint_shift;
-  const int groups = ((blocks - 1) >> b.hint_shift) + 1;
-  for (int g = 0, run = 0; g < groups; ++g) {
-    while (run + 1 < b.count && b.first_block[run + 1] <= g << b.hint_shift) ++run;
-    b.hint[g] = run;
-  }
-  b.hint[groups] = b.count - 1;
-}
 
 enum : int32_t {
   kRedPreMul = 1,      // every contribution * pre, rounded to the reduce dtype
@@ -573,6 +594,20 @@ __device__ __forceinline__ auto run_from_hint(const int32_t* first_block, const 
   }
   return make(blk - begin, end - begin, r, h);
 }
+
+struct InPlaceView {
+  const InPlaceBatch& t;
+  __device__ __forceinline__ int block() const { return int(blockIdx.x); }
+  __device__ __forceinline__ SpanRun span_run(int blk) const {
+    const int g = blk >> t.hint_shift;
+    int s = t.hint[g];
+    const int hi = t.hint[g + 1];
+    if (hi > s) s = find_run_in(t.first_block, s, hi + 1, blk);
+    const uint32_t nh = t.numel_head[s];
+    return {blk - t.first_block[s], t.first_block[s + 1] - t.first_block[s], t.data[s], t.data[s],
+            int64_t(nh & ((1u << kNumelBits) - 1)), int32_t(nh >> kNumelBits) - 1};
+  }
+};
 
 struct PieceArgView {
   const PieceBatch& t;

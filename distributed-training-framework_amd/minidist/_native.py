@@ -25,7 +25,7 @@ MDX_F32 = 0
 MDX_BF16 = 1
 MDX_F16 = 2
 MDX_MAX_WORLD = 16
-ABI_VERSION = 10
+ABI_VERSION = 11
 # Reduction operations of mdx_allreduce_op (torch.distributed.ReduceOp's SUM, PRODUCT, MIN, MAX).
 MDX_OP_SUM, MDX_OP_PRODUCT, MDX_OP_MIN, MDX_OP_MAX = 0, 1, 2, 3
 
@@ -35,6 +35,7 @@ SIGNATURES: dict[str, tuple] = {
     "mdx_pack": (_i32, [_vp, _i32, _i32, _i32, _f32, _i32, _vp, _vp]),
     "mdx_unpack": (_i32, [_vp, _i32, _i32, _i32, _f32, _vp, _vp]),
     "mdx_unscale_found_inf": (_i32, [_vp, _i32, _i32, _f32, _vp, _vp]),
+    "mdx_unscale_found_inf_clear": (_i32, [_vp, _i32, _i32, _f32, _vp, _vp, _vp]),
     "mdx_allreduce_sum": (_i32, [_vp, _i32, _i32, _vp, _vp, _i32, _vp, _vp]),
     "mdx_allreduce_op": (_i32, [_vp, _i32, _i32, _i32, _vp, _vp, _i32, _vp, _vp]),
     "mdx_allreduce_unpack": (_i32, [_vp, _i32, _i32, _vp, _i32, _vp, _i32, _f32, _vp, _vp]),
@@ -216,9 +217,11 @@ def unpack(
     check(rc, "mdx_unpack")
 
 
-def unscale_found_inf(spans: np.ndarray, dtype: int, inv_scale: float, found_inf: int | None, stream: int) -> None:
-    rc = lib().mdx_unscale_found_inf(_ptr(spans), len(spans), dtype, inv_scale, found_inf, stream)
-    check(rc, "mdx_unscale_found_inf")
+def unscale_found_inf(
+    spans: np.ndarray, dtype: int, inv_scale: float, found_inf: int | None, stream: int, clear_flag: int | None = None
+) -> None:
+    rc = lib().mdx_unscale_found_inf_clear(_ptr(spans), len(spans), dtype, inv_scale, found_inf, clear_flag, stream)
+    check(rc, "mdx_unscale_found_inf_clear")
 
 
 def allreduce_sum(

@@ -5,7 +5,7 @@ Same surface and arithmetic as the reference's minidist/amp.py
 ``DistributedGradScaler`` :114-267).  ``unscale_`` is where the data path
 changes: instead of ~6 ATen launches per gradient tensor (``mul_``,
 ``isfinite``, ``~``, ``any``, ``to``, ``+=``, amp.py:208-213) it issues one
-multi-tensor ``mdx_unscale_found_inf`` dispatch per dtype, whose waves store
+multi-tensor ``mdx_unscale_found_inf_clear`` dispatch per dtype, whose waves store
 a 1 into a flag when they produce a non-finite value.  Gradients that
 a DDP wrapper already unscaled in its unpack epilogue (``grad_scaler=``) are
 skipped.  The flag is then all-reduced with MAX across a real process group
@@ -295,10 +295,17 @@ class DistributedGradScaler:
                     raise RuntimeError("unscale_: gradient is not contiguous")
                 groups.setdefault(g.dtype, []).append((g.data_ptr(), g.data_ptr(), g.numel()))
         stream = _native.stream_of(flag.device)
+        # The first dispatch also clears the next step's flag, unless a fused producer's did.
+        clear = None
+        if groups and device not in self._next_armed:
+            clear = self._next_flag(device).data_ptr()
         for dtype, rows in groups.items():
             _native.unscale_found_inf(
-                _native.spans_array(rows), _native.dtype_code(dtype), inv_scale, flag.data_ptr(), stream
+                _native.spans_array(rows), _native.dtype_code(dtype), inv_scale, flag.data_ptr(), stream, clear
             )
+            if clear is not None:
+                clear = None
+                self._next_flag_cleared(device)
 
         if isinstance(flag, _HostFlag):
             flag.settle()

@@ -41,7 +41,7 @@
 extern "C" {
 #endif
 
-#define MDX_ABI_VERSION 10
+#define MDX_ABI_VERSION 11
 
 /* Only the entry points below are exported (the library builds with hidden
  * visibility by default). */
@@ -125,6 +125,15 @@ MDX_API int mdx_unpack(const mdx_span* spans, int n_spans, int src_dtype, int ds
  * g = rnd(g * inv_scale); flag if !isfinite(g). */
 MDX_API int mdx_unscale_found_inf(const mdx_span* spans, int n_spans, int dtype, float inv_scale,
                           int32_t* found_inf, void* stream);
+
+/* mdx_unscale_found_inf, whose first dispatch also sets `clear_flag` (may be
+ * NULL, must differ from found_inf) to 0: the loss scaler's flag for the NEXT
+ * step, which nothing reads or sets during this one, as in
+ * mdx_pack_allreduce_unpack.  It is cleared even when there is nothing to
+ * unscale.  Replaces, with the loop above, the per-step
+ * `found_inf = zeros(1)` (minidist/amp.py:206). */
+MDX_API int mdx_unscale_found_inf_clear(const mdx_span* spans, int n_spans, int dtype, float inv_scale,
+                                        int32_t* found_inf, int32_t* clear_flag, void* stream);
 
 /* W-way SUM all-reduce arithmetic over W replica buffers resident in HBM,
  * in the fixed rank order ((in[0] + in[1]) + in[2]) + ..., one rounding per

@@ -204,6 +204,37 @@ def test_unscale_in_place_matches_oracle(rng, dt):
     assert bool(flag.item()) == found
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("n", [0, 1, 224, 225, 500])
+@pytest.mark.parametrize("inv_scale", [1.0, 2.0**-4])
+def test_unscale_many_runs_and_flag_clear(rng, dt, n, inv_scale):
+    """In-place tables of up to 224 runs: none, one, a full table, one run more and three tables, with
+    long runs between one-workgroup ones at odd offsets; the first dispatch clears the other flag."""
+    sizes = [30_001 if k % 60 == 7 else int(x) for k, x in enumerate(rng.integers(0, 700, n))]
+    shifts = rng.integers(0, 8, n)
+    hosts = [values(rng, s, dt, specials=k % 100 == 99) for k, s in enumerate(sizes)]
+    devs = [to_dev(np.concatenate([o.zeros(int(h), dt), v])) for h, v in zip(shifts, hosts)]
+    rows = [(0, t.data_ptr() + int(h) * esize(dt), s) for t, h, s in zip(devs, shifts, sizes)]
+    flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+    other = torch.ones(1, dtype=torch.int32, device=DEV)
+    nat.unscale_found_inf(nat.spans_array(rows), code(dt), nat.f32(inv_scale), flag.data_ptr(), stream(),
+                          other.data_ptr())
+    found = False
+    for t, h, v in zip(devs, shifts, hosts):
+        want = o.mul_scalar(v, dt, inv_scale) if inv_scale != 1.0 else v
+        found |= bool((~o.isfinite(want, dt)).any())
+        got = to_host(t)
+        assert same_bits(got[int(h):], want), first_mismatch(got[int(h):], want)
+        assert not np.any(got[: int(h)])
+    assert bool(flag.item()) == found and other.item() == 0
+
+
+def test_unscale_rejects_clearing_its_own_flag():
+    flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+    with pytest.raises(RuntimeError, match="overlap"):
+        nat.unscale_found_inf(nat.spans_array([]), nat.MDX_F32, 0.5, flag.data_ptr(), stream(), flag.data_ptr())
+
+
 # ---------------------------------------------------------------------------
 # W-way all-reduce
 # ---------------------------------------------------------------------------
