@@ -187,6 +187,37 @@ int run_copy(const mdx_span* spans, int n_spans, int sdt, int ddt, const CopyPar
   return p.clear != nullptr ? status(launch_clear_flag(p.clear, stream)) : MDX_OK;
 }
 
+// The first `n_first` spans from dtype `sdt`, the others from `ddt`: one dispatch
+// where all their runs fit one table, otherwise the casts and then the copies.
+int run_gather(const mdx_span* spans, int n_spans, int n_first, int sdt, int ddt, const CopyParams& p,
+               hipStream_t stream) {
+  int runs = 0;
+  for (int i = 0; i < n_spans; ++i) runs += int(std::min<int64_t>(kRunsPerLaunch, ceil_div(spans[i].numel, kMaxRunElems)));
+  if (sdt == ddt) return run_copy(spans, n_spans, ddt, ddt, p, stream);
+  if (runs == 0 || runs > kRunsPerLaunch) {
+    const int rc = run_copy(spans, n_first, sdt, ddt, p, stream);
+    CopyParams rest = p;
+    rest.clear = nullptr;  // cleared by the call above
+    return rc != MDX_OK ? rc : run_copy(spans + n_first, n_spans - n_first, ddt, ddt, rest, stream);
+  }
+  SpanBatch b;
+  memset(&b, 0, sizeof(b));
+  auto push = [&](const Rec& r) -> int {
+    const int k = b.count;
+    b.src[k] = r.a;
+    b.dst[k] = r.b;
+    b.numel[k] = r.numel;
+    b.head[k] = r.head;
+    b.first_block[k + 1] = b.first_block[k] + r.blocks;
+    b.count = k + 1;
+    return MDX_OK;
+  };
+  for_each_span_run(spans, n_first, sdt, ddt, false, push);
+  const int cast_blocks = b.first_block[b.count];
+  for_each_span_run(spans + n_first, n_spans - n_first, ddt, ddt, false, push);
+  return status(launch_gather(sdt, ddt, b, cast_blocks, p, stream));
+}
+
 // The in-place form (each span's `dst` alone), with a table of its own.
 int run_in_place(const mdx_span* spans, int n_spans, int dt, const CopyParams& params, hipStream_t stream) {
   InPlaceBatch b;
@@ -703,9 +734,17 @@ const char* mdx_strerror(int code) {
 
 int mdx_pack(const mdx_span* spans, int n_spans, int src_dtype, int dst_dtype, float scale,
              int divide, int32_t* clear_flag, void* stream) {
+  const int n_first = src_dtype >> 8;  // MDX_MIXED, or 0
+  if (n_first > 0) src_dtype &= 0xff;
   if (!valid_dtype(src_dtype) || !valid_dtype(dst_dtype)) return MDX_EDTYPE;
   int rc = check_spans(spans, n_spans, false);
   if (rc != MDX_OK) return rc;
+  if (n_first > 0) {
+    if (scale != 1.0f) return MDX_EDTYPE;
+    if (n_first > n_spans) return MDX_EINVAL;
+    return run_gather(spans, n_spans, n_first, src_dtype, dst_dtype, CopyParams{1.0f, 0, nullptr, clear_flag},
+                      static_cast<hipStream_t>(stream));
+  }
   int32_t flags = 0;
   if (scale != 1.0f) flags = divide ? kCopyDivide : kCopyScale;
   CopyParams p{scale, flags, nullptr, clear_flag};

@@ -320,6 +320,9 @@ constexpr int kHeadRange = 8;
 
 hipError_t launch_copy(int src_dtype, int dst_dtype, const SpanBatch& b, const CopyParams& p,
                        hipStream_t stream);
+// A cast of the first `cast_blocks` workgroups' spans and a copy of the others'.
+hipError_t launch_gather(int src_dtype, int dst_dtype, const SpanBatch& b, int cast_blocks, const CopyParams& p,
+                         hipStream_t stream);
 hipError_t launch_unscale(int dtype, const InPlaceBatch& b, const CopyParams& p, hipStream_t stream);
 hipError_t launch_clear_flag(int32_t* flag, hipStream_t stream);
 int copy_frag_elems(int src_dtype, int dst_dtype);

@@ -140,6 +140,11 @@ def dtype_code(dtype: torch.dtype) -> int:
     raise TypeError(f"minidist kernels handle float32, bfloat16 and float16, not {dtype}")
 
 
+def mixed_code(first: int, n_first: int) -> int:
+    """``MDX_MIXED``: the source dtype code of a :func:`pack` whose first ``n_first`` spans hold ``first``."""
+    return first | (n_first << 8)
+
+
 def require_device_tensor(t: torch.Tensor, what: str) -> None:
     if not t.is_cuda:
         raise RuntimeError(

@@ -88,6 +88,14 @@ def _copy_spans(rows, src_dtype: torch.dtype, dst_dtype: torch.dtype, device: to
         )
 
 
+def _gather_spans(casts, copies, src_dtype: torch.dtype, dtype: torch.dtype, device: torch.device) -> None:
+    """Master shards cast from ``src_dtype`` into their slots and peers' shards copied into theirs, in
+    one dispatch (where the spans fit one kernel-argument table)."""
+    code = _native.dtype_code(dtype)
+    src = code if src_dtype == dtype else _native.mixed_code(_native.dtype_code(src_dtype), len(casts))
+    _native.pack(_native.spans_array([*casts, *copies]), src, code, 1.0, False, _native.stream_of(device))
+
+
 def _emulates_peers(group) -> bool:
     """A ResidentGroup whose peers are staged in this process (an IpcGroup's are processes)."""
     return isinstance(group, comm.ResidentGroup) and not isinstance(group, comm.IpcGroup)
@@ -331,14 +339,15 @@ class _FSDPUnit:
         """(master shard, this rank's slot of the gather buffer, S): the unshard cast."""
         self._require_gathered_storage()
         S = self.shard_numel
-        return (self.flat_shard.detach().data_ptr(), self._full[self.rank * S :].data_ptr(), S)
+        return (self.flat_shard.data_ptr(), self._full.data_ptr() + self.rank * S * self._full.element_size(), S)
 
     def _peer_slot_spans(self) -> list[tuple[int, int, int]]:
         """(peer's gathered shard, its slot, S) for every peer (ResidentGroup): the all-gather."""
         self._require_gathered_storage()
-        S = self.shard_numel
-        return [(self._peer_shards[r].data_ptr(), self._full[r * S :].data_ptr(), S)
-                for r in range(self.world) if r != self.rank]
+        # both are rows of S elements of the gathered dtype, one after another
+        S, step = self.shard_numel, self.shard_numel * self._full.element_size()
+        src, dst = self._peer_shards.data_ptr(), self._full.data_ptr()
+        return [(src + r * step, dst + r * step, S) for r in range(self.world) if r != self.rank]
 
     def _account_all_gather(self) -> None:
         if self.world > 1:
@@ -346,14 +355,17 @@ class _FSDPUnit:
             comm.comm_stats.add("all_gather", payload, int((self.world - 1) / self.world * payload))
 
     def _gather_now(self) -> None:
+        if self._peer_shards is not None:
+            self._account_all_gather()
+            _gather_spans([self._own_slot_span()], self._peer_slot_spans(), self.flat_shard.dtype, self._full.dtype,
+                          self.device)
+            return
         self._cast_own_slot_now()
         S = self.shard_numel
         if self.world > 1:
             self._account_all_gather()
             if self._ipc is not None:
                 self._gather_over_ipc()
-            elif isinstance(self.group, comm.ResidentGroup):
-                _copy_spans(self._peer_slot_spans(), self._full.dtype, self._full.dtype, self.device)
             else:
                 own = self._full[self.rank * S : (self.rank + 1) * S]
                 comm.dist_all_gather_into_tensor(self._full, own, group=self.group)
@@ -873,6 +885,13 @@ class FullyShardedDataParallel(nn.Module):
             by_dtype: dict[tuple[torch.dtype, torch.dtype], list] = {}
             for u in units:
                 by_dtype.setdefault((u.flat_shard.dtype, u._full.dtype), []).append(u._own_slot_span())
+            if resident and not ipc and len(by_dtype) == 1 and len(units) * self.world_size <= _KERNARG_RUNS:
+                ((src, dst), casts), = by_dtype.items()
+                for u in units:
+                    u._account_all_gather()
+                peers = [] if self.world_size == 1 else [span for u in units for span in u._peer_slot_spans()]
+                _gather_spans(casts, peers, src, dst, units[0].device)
+                return
             for (src, dst), spans in by_dtype.items():
                 self._copy_many("cast", spans, src, dst)
             if ipc:

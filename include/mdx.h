@@ -56,6 +56,9 @@ extern "C" {
  * except where stated. */
 enum { MDX_F32 = 0, MDX_BF16 = 1, MDX_F16 = 2 };
 
+/* A source dtype code for mdx_pack: the first `n_first` spans hold `dtype`. */
+#define MDX_MIXED(dtype, n_first) ((dtype) | ((n_first) << 8))
+
 /* Status codes (negative; positive values are hipError_t). */
 enum {
   MDX_OK = 0,
@@ -99,7 +102,11 @@ typedef struct mdx_piece {
  * `buf[off:off+n].copy_(p.grad.reshape(-1))` then `buf.div_(W)`
  * (minidist/fsdp.py:218-227), with scale = W and divide = 1.
  * dst[i] = rnd_dst(rnd_dst(src[i]) * scale), or ... / scale when divide != 0;
- * the scaling is skipped when scale == 1.  All spans of one call share dtypes.
+ * the scaling is skipped when scale == 1.  All spans of one call share dtypes,
+ * except that `src_dtype` may be MDX_MIXED(d, n): the first n spans are read as
+ * dtype d, the others as dst_dtype (scale 1 only, else MDX_EDTYPE).  That is one
+ * FSDP unit's gather in one dispatch (minidist/fsdp.py:172-182): the master
+ * shard cast into this rank's slot, the peers' gathered shards copied into theirs.
  * `clear_flag` (may be NULL): a found-inf flag (int32, device memory) that the
  * call also sets to 0, ordered on `stream` like the copy -- the scaler's
  * once-per-step clear (minidist/amp.py:206 `found_inf = zeros(1)`) folded into

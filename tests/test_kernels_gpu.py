@@ -204,6 +204,41 @@ def test_unscale_in_place_matches_oracle(rng, dt):
     assert bool(flag.item()) == found
 
 
+@pytest.mark.parametrize("sdt", DTYPES)
+@pytest.mark.parametrize("ddt", DTYPES)
+@pytest.mark.parametrize("n_casts,n_copies", [(1, 0), (1, 7), (3, 1), (8, 40), (20, 40)])
+def test_pack_mixed_sources_matches_oracle(rng, sdt, ddt, n_casts, n_copies):
+    """The first spans from one dtype and the others from the destination's, in one dispatch (up to 48
+    spans) or a cast and a copy dispatch, with empty, ragged and misaligned spans and a flag clear."""
+    sizes = [[0, 1, 7, 300, 4096, 12345, 20001][int(k)] for k in rng.integers(0, 7, n_casts + n_copies)]
+    dst = empty_dev(sum(sizes) + 3 * len(sizes), ddt)
+    want = to_host(dst)
+    rows, keep, off = [], [], 0
+    for k, n in enumerate(sizes):
+        dt, shift = sdt if k < n_casts else ddt, int(rng.integers(0, 4))
+        host = values(rng, n, dt)
+        t = to_dev(np.concatenate([o.zeros(shift, dt), host]))
+        null = k % 9 == 8
+        off += int(rng.integers(0, 3))
+        rows.append((0 if null else t.data_ptr() + shift * esize(dt), dst.data_ptr() + off * esize(ddt), n))
+        want[off : off + n] = o.zeros(n, ddt) if null else o.convert(host, dt, ddt)
+        off += n
+        keep.append(t)
+    flag = torch.ones(1, dtype=torch.int32, device=DEV)
+    nat.pack(nat.spans_array(rows), nat.mixed_code(code(sdt), n_casts), code(ddt), 1.0, False, stream(),
+             flag.data_ptr())
+    got = to_host(dst)
+    assert same_bits(got, want), first_mismatch(got, want)
+    assert flag.item() == 0
+
+
+def test_pack_mixed_sources_rejects():
+    spans = nat.spans_array([(64, 128, 0)])
+    for src, scale in [(nat.mixed_code(0, 2), 1.0), (nat.mixed_code(0, 1), 0.5), (nat.mixed_code(5, 1), 1.0)]:
+        with pytest.raises(RuntimeError, match="mdx_pack failed"):
+            nat.pack(spans, src, 1, scale, False, stream())
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("n", [0, 1, 224, 225, 500])
 @pytest.mark.parametrize("inv_scale", [1.0, 2.0**-4])
