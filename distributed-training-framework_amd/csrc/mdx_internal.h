@@ -314,10 +314,6 @@ constexpr int copy_unroll(int frag_in_bytes) { return frag_in_bytes >= 16 ? 1 : 
 constexpr int copy_unroll_of(int src_size, int dst_size) {
   return src_size > dst_size ? 2 : copy_unroll(copy_frag_elems_of(src_size, dst_size) * src_size);
 }
-// Alignment heads are searched over 16 bytes of the narrowest (2-byte) type,
-// whatever the fragment, so that mixed-dtype runs keep a vector body.
-constexpr int kHeadRange = 8;
-
 hipError_t launch_copy(int src_dtype, int dst_dtype, const SpanBatch& b, const CopyParams& p,
                        hipStream_t stream);
 // A cast of the first `cast_blocks` workgroups' spans and a copy of the others'.

@@ -730,6 +730,37 @@ def test_plan_run_hints_resolve_every_workgroup(seed):
     assert np.array_equal(got, brute)
 
 
+@pytest.mark.parametrize("seed", range(4))
+def test_run_heads_align_the_most_streams(seed):
+    """A run's head against brute force over every element offset: no other offset 16-byte aligns more
+    of the streams (the stored one counts double), and of those none puts more at a 128-byte line; a
+    run under 4096 elements is only aligned to 16 bytes, and one with no fragment after it has none."""
+    rng = np.random.default_rng(100 + seed)
+    L = nat.lib()
+    for _ in range(100):
+        sdt, ddt = [(0, 0), (1, 1), (0, 1), (2, 0)][int(rng.integers(4))]
+        ss, ds = (4 if d == 0 else 2 for d in (sdt, ddt))
+        n = [1, 3, 9, 70, 4095, 4096, 100_000][int(rng.integers(7))]
+        dst = (1 << 40) + ds * int(rng.integers(0, 4096 // ds))
+        src = (1 << 41) + ss * int(rng.integers(0, 4096 // ss))
+        if rng.random() < 0.3:
+            src = (1 << 41) + (dst & 127) * ss // ds  # streams that can share a boundary
+        spans = nat.spans_array([(src, dst, n)])
+        size = ctypes.c_int64(0)
+        assert L.mdx_plan_spans(spans.ctypes.data, 1, sdt, ddt, None, ctypes.byref(size)) == nat.MDX_ESIZE
+        buf = np.zeros((size.value + 7) // 8, dtype=np.uint64)
+        assert L.mdx_plan_spans(spans.ctypes.data, 1, sdt, ddt, buf.ctypes.data, ctypes.byref(size)) == 0
+        off = int(buf.view(np.int64)[24])  # the header's offset of the heads, after the run boundaries'
+        head = int(buf.view(np.uint8)[off : off + 4].view(np.int32)[0])
+
+        def score(h, bound):
+            return 2 * ((dst + h * ds) % bound == 0) + ((src + h * ss) % bound == 0)
+
+        line = 128 if n >= 4096 else 16
+        best = max(range(line // 2), key=lambda h: (score(h, 16), score(h, line), -h))
+        assert head == (best if n >= best + 16 // max(ss, ds) else -1), (src, dst, n, sdt, ddt)
+
+
 @pytest.mark.parametrize("seed", [0, 1])
 def test_plan_builders_on_random_tables(seed):
     """Every plan builder on random tables (fake device addresses, aligned or not, runs from empty to
