@@ -447,6 +447,32 @@ def test_reduce_scatter_share_width_classes(rng, idt, rdt, sdt, W, rank, accumul
     _share_case(rng, [4100 * W + 3, 517 * W, 6, 1031 * W + 1], idt, rdt, sdt, W, rank, accumulate)
 
 
+@pytest.mark.parametrize("W", [3, 5, 6, 7, 9, 10, 11, 12, 13, 14, 15])
+@pytest.mark.parametrize("idt,rdt", [(o.BF16, o.F32), (o.F16, o.F32), (o.BF16, o.BF16), (o.F16, o.F16), (o.F32, o.F32)])
+def test_reduce_scatter_share_division(rng, W, idt, rdt):
+    """x / W for every W that is not a power of two: rank 0's contribution runs through every 16-bit
+    pattern (fp32: random patterns, every exponent, and the edges of the exact quotient's range), the
+    others are -0, so the shard is the quotient itself, bit for bit the oracle's."""
+    if idt == o.F32:
+        bits = rng.integers(0, 2**32, 1 << 18, dtype=np.uint64).astype(np.uint32)
+        edges = np.array([e << 23 for e in range(256)], np.uint32)
+        edges = np.concatenate([edges, edges + 1, edges - 1, edges | np.uint32(0x80000000)])
+        own = np.concatenate([bits, np.tile(edges, 8)]).view(np.float32)
+    else:
+        own = np.arange(1 << 16, dtype=np.uint16)
+        rng.shuffle(own[: 1 << 15])  # half of the waves meet specials, half none
+        own = own.view(np.float16) if idt == o.F16 else own
+    n = own.size
+    minus = o.from_f32(np.full(n, -0.0, np.float32), idt)
+    dev, peer, shard = to_dev(own), to_dev(minus), empty_dev(n, rdt)
+    nat.reduce_scatter_share(nat.pieces_array([(dev.data_ptr(), 0, n)]), [0] + [peer.data_ptr()] * (W - 1), 0,
+                             code(idt), code(rdt), True, shard.data_ptr(), code(rdt), False, 1.0, None, stream())
+    want = o.div_scalar(o.convert(own, idt, rdt), rdt, W)
+    rest = o.div_scalar(o.convert(minus, idt, rdt), rdt, W)
+    want = o.allreduce_sum([want] + [rest] * (W - 1), rdt)
+    assert same_bits(to_host(shard), want), first_mismatch(to_host(shard), want)
+
+
 @pytest.mark.parametrize("seed", range(40))
 def test_reduce_scatter_share_fuzz(seed):
     """Seeded random shares: 1-10 parameters of 1-5000 elements, W in [2, 16], any rank, fp32 / bf16 /
