@@ -26,6 +26,7 @@ inline int status(hipError_t e) { return e == hipSuccess ? MDX_OK : int(e); }
 // Runs from this length on are aligned to 128-byte lines (a head of at most 63
 // elements, one per lane of the run's first wave), shorter ones to 16 bytes.
 constexpr int64_t kLineHeadMinElems = 4096;
+static_assert(128 / 2 - 1 <= kMaxHead, "a line's worth of 2-byte elements less one");
 
 inline uintptr_t addr(const void* p) { return reinterpret_cast<uintptr_t>(p); }
 
@@ -125,8 +126,9 @@ int for_each_span_run(const mdx_span* spans, int n_spans, int sdt, int ddt, bool
     const mdx_span& sp = spans[i];
     const char* src = static_cast<const char*>(in_place ? sp.dst : sp.src);
     char* dst = static_cast<char*>(sp.dst);
-    for (int64_t done = 0; done < sp.numel; done += kMaxRunElems) {
-      const int64_t n = std::min<int64_t>(kMaxRunElems, sp.numel - done);
+    const int64_t max_run = in_place ? kMaxInPlaceRunElems : kMaxRunElems;
+    for (int64_t done = 0; done < sp.numel; done += max_run) {
+      const int64_t n = std::min<int64_t>(max_run, sp.numel - done);
       const void* rs = src ? src + done * ss : nullptr;
       void* rd = dst + done * ds;
       uintptr_t ptrs[2];

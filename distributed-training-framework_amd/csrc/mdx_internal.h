@@ -21,6 +21,7 @@ namespace mdx {
 constexpr int kBlock = 64;  // one wave64 per workgroup (measured: beats 128, 256, 512 and 1024 lanes)
 constexpr int kRunsPerLaunch = 48;        // runs per dispatch (kernarg budget)
 constexpr int64_t kMaxRunElems = int64_t(1) << 26;
+constexpr int kMaxHead = kBlock - 1;  // elements before a run's vector body: one per lane of one wave
 
 // bf16 and fp16 storage types: raw bits, so that conversions are exact and
 // explicit.
@@ -257,7 +258,7 @@ struct SpanBatch {
   const void* src[kRunsPerLaunch];
   void* dst[kRunsPerLaunch];
   int64_t numel[kRunsPerLaunch];
-  int32_t head[kRunsPerLaunch];  // scalar elements before the 16B-aligned body; -1 = no body
+  int32_t head[kRunsPerLaunch];  // scalar elements before the vector body, at most kMaxHead; -1 = no body
   int32_t first_block[kRunsPerLaunch + 1];
   int32_t count;
 };
@@ -286,8 +287,10 @@ struct InPlaceBatch {
   int32_t hint_shift;
   int32_t hint[kArgHintGroups + 1];
 };
-constexpr int kNumelBits = 27;
-static_assert(kMaxRunElems < (int64_t(1) << kNumelBits), "a run's length fits its field");
+constexpr int64_t kMaxInPlaceRunElems = int64_t(1) << 24;
+constexpr int kNumelBits = 25;
+static_assert(kMaxInPlaceRunElems < (int64_t(1) << kNumelBits), "a run's length fits its field");
+static_assert(kMaxHead + 1 < (1 << (32 - kNumelBits)), "and its head the bits above");
 static_assert(sizeof(InPlaceBatch) + sizeof(CopyParams) <= 4096, "one dispatch's kernel arguments");
 
 // Fragments.  In the W-way reductions a fragment is one 16-byte vector of the

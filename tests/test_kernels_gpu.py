@@ -244,9 +244,13 @@ def test_pack_mixed_sources_rejects():
 @pytest.mark.parametrize("inv_scale", [1.0, 2.0**-4])
 def test_unscale_many_runs_and_flag_clear(rng, dt, n, inv_scale):
     """In-place tables of up to 224 runs: none, one, a full table, one run more and three tables, with
-    long runs between one-workgroup ones at odd offsets; the first dispatch clears the other flag."""
-    sizes = [30_001 if k % 60 == 7 else int(x) for k, x in enumerate(rng.integers(0, 700, n))]
+    runs of a long head and whole chunks (a head read wrong leaves their end out) between one-workgroup
+    ones at odd offsets; the first dispatch clears the other flag."""
     shifts = rng.integers(0, 8, n)
+    sizes = [int(x) for x in rng.integers(0, 700, n)]
+    per_line = 128 // esize(dt)
+    for k in range(n // 2, n, 30):  # a head of up to a line less one element, then whole chunks and no more
+        sizes[k] = (per_line - int(shifts[k])) % per_line + 64 * (16 // esize(dt)) * 9
     hosts = [values(rng, s, dt, specials=k % 100 == 99) for k, s in enumerate(sizes)]
     devs = [to_dev(np.concatenate([o.zeros(int(h), dt), v])) for h, v in zip(shifts, hosts)]
     rows = [(0, t.data_ptr() + int(h) * esize(dt), s) for t, h, s in zip(devs, shifts, sizes)]
@@ -262,6 +266,17 @@ def test_unscale_many_runs_and_flag_clear(rng, dt, n, inv_scale):
         assert same_bits(got[int(h):], want), first_mismatch(got[int(h):], want)
         assert not np.any(got[: int(h)])
     assert bool(flag.item()) == found and other.item() == 0
+
+
+def test_unscale_run_past_the_in_place_limit():
+    """A gradient of more than 2^24 elements is cut into runs that line up."""
+    n = (1 << 24) + 777
+    t = torch.arange(n + 1, dtype=torch.float32, device=DEV).remainder_(4096.0)
+    want = t.clone()
+    want[1:] *= 0.25  # exact
+    flag = torch.zeros(1, dtype=torch.int32, device=DEV)
+    nat.unscale_found_inf(nat.spans_array([(0, t.data_ptr() + 4, n)]), nat.MDX_F32, 0.25, flag.data_ptr(), stream())
+    assert torch.equal(t, want) and flag.item() == 0
 
 
 def test_unscale_rejects_clearing_its_own_flag():
