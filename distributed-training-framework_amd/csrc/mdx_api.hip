@@ -392,7 +392,7 @@ int build_plan(PlanHeader proto, Gen&& gen, void* plan, int64_t* plan_bytes) {
 int plan_view(const void* plan, const void* d_plan, int32_t kind, const PlanHeader** hdr, DevTable* t) {
   if (plan == nullptr || d_plan == nullptr) return MDX_EINVAL;
   const PlanHeader* h = static_cast<const PlanHeader*>(plan);
-  if (h->magic != kPlanMagic || h->kind != kind) return MDX_EINVAL;
+  if (h->magic != kPlanMagic || h->kind != kind || h->columns[0] != 0) return MDX_EINVAL;
   const char* d = static_cast<const char*>(d_plan);
   t->first_block = reinterpret_cast<const int32_t*>(d + h->off_first_block);
   t->head = reinterpret_cast<const int32_t*>(d + h->off_head);
@@ -731,7 +731,7 @@ bool plan_layout_matches(const PlanHeader* h) {
   PlanHeader ref = *h;
   plan_layout(&ref, h->count, h->blocks);
   return ref.bytes == h->bytes && ref.off_first_block == h->off_first_block && ref.off_head == h->off_head &&
-         ref.off_run == h->off_run && ref.off_hint == h->off_hint;
+         ref.off_run == h->off_run && ref.off_hint == h->off_hint && h->columns[0] == 0;
 }
 
 // The device `stream` runs on, which must be the current one.

@@ -769,7 +769,7 @@ struct PlanHeader {
   uint64_t replicas[MDX_MAX_WORLD];
   uint64_t out;
   int64_t off_first_block, off_head, off_run;
-  int64_t unused[3];
+  int64_t columns[3];  // 0: a plan whose runs are columns (a library before ABI 11) has offsets here and is refused
   int64_t bytes;
   int64_t off_hint;
 };

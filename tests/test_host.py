@@ -857,6 +857,20 @@ def test_planned_launch_rejects_bad_plans_before_launch():
     assert L.mdx_allreduce_unpack_planned(junk.ctypes.data, junk.ctypes.data, 1.0, None, None) == -1  # wrong kind
 
 
+def test_planned_launch_rejects_a_plan_of_columns():
+    """A plan that an earlier library built (its runs as columns, their offsets in the header) has the
+    same magic, kinds and size as one of run records; no launch takes it for one."""
+    L = nat.lib()
+    buf = np.zeros(4096, dtype=np.uint64)
+    size = ctypes.c_int64(buf.nbytes)
+    spans = nat.spans_array([(0x10000000, 0x40000000, 64)])
+    assert L.mdx_plan_spans(spans.ctypes.data, 1, 0, 0, buf.ctypes.data, ctypes.byref(size)) == 0
+    assert buf[26] == 0
+    buf[26] = 256
+    assert L.mdx_pack_planned(buf.ctypes.data, buf.ctypes.data, 1.0, 0, None, None) == -1
+    assert L.mdx_unpack_planned(buf.ctypes.data, buf.ctypes.data, 1.0, None, None) == -1
+
+
 def test_bench_refuses_more_than_one_gpu():
     """bench.py measures one GPU: --gpus N > 1 exits (code 2) with a message that says so,
     before anything touches a GPU."""
