@@ -209,6 +209,9 @@ class _FSDPUnit:
         # Pad so the flat parameter divides evenly (fsdp.py:132-136).
         self.shard_numel = (self.total_numel + self.world - 1) // self.world
         self.padded_numel = self.shard_numel * self.world
+        # Laid out once: walking every parameter of a unit for its share on each step was a sixth of
+        # the host time that a step of many small units waits for.
+        self._parts, self._padding = self._shard_pieces()
 
         src_dtype = params[0].dtype
         shard_dtype = policy.param_dtype if policy.keep_low_precision_shard else src_dtype
@@ -425,24 +428,32 @@ class _FSDPUnit:
         """Whether any parameter still has a full-size gradient (left by a ``no_sync`` backward)."""
         return any(p.grad is not None for p in self.params)
 
-    def _own_pieces(self) -> list[tuple[int, int, int]]:
-        """(own grad address | 0, shard position, numel) covering the whole shard."""
-        S, lo = self.shard_numel, self.rank * self.shard_numel
-        hi = lo + S
-        rows, cursor, off = [], lo, 0
-        for p, n in zip(self.params, self.numels, strict=True):
+    def _shard_pieces(self) -> tuple[list[tuple[int, int, int, int]], tuple[int, int] | None]:
+        """What this rank's shard is made of, fixed when the unit is built: (parameter index, first
+        element of it, shard position, numel) of each part, and the padding's (position, numel)."""
+        lo = self.rank * self.shard_numel
+        hi = lo + self.shard_numel
+        parts, cursor, off = [], lo, 0
+        for k, n in enumerate(self.numels):
             a, b = max(off, lo), min(off + n, hi)
             if a < b:
-                g = p.grad
-                if g is None:
-                    rows.append((0, a - lo, b - a))
-                else:
-                    _check_grad(g)
-                    rows.append((g.data_ptr() + (a - off) * g.element_size(), a - lo, b - a))
+                parts.append((k, a - off, a - lo, b - a))
                 cursor = b
             off += n
-        if cursor < hi:  # padding at the end of the last shard
-            rows.append((0, cursor - lo, hi - cursor))
+        return parts, (cursor - lo, hi - cursor) if cursor < hi else None  # at the end of the last shards
+
+    def _own_pieces(self) -> list[tuple[int, int, int]]:
+        """(own grad address | 0, shard position, numel) covering the whole shard."""
+        params, rows = self.params, []
+        for k, first, pos, n in self._parts:
+            g = params[k].grad
+            if g is None:
+                rows.append((0, pos, n))
+            else:
+                _check_grad(g)
+                rows.append((g.data_ptr() + first * g.element_size(), pos, n))
+        if self._padding is not None:
+            rows.append((0, *self._padding))
         return rows
 
     def _grad_out(self) -> tuple[torch.Tensor, bool]:
@@ -526,7 +537,7 @@ class _FSDPUnit:
 
     def _account_reduce_scatter(self) -> None:
         if self.world > 1:
-            payload = self.padded_numel * torch.empty((), dtype=self.policy.reduce_dtype).element_size()
+            payload = self.padded_numel * self.policy.reduce_dtype.itemsize
             comm.comm_stats.add("reduce_scatter", payload, int((self.world - 1) / self.world * payload))
 
     def _finish_reduce_scatter(self, out: torch.Tensor, accumulate: bool) -> None:
