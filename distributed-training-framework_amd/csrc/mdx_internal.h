@@ -711,6 +711,54 @@ struct PieceFewView {
   }
 };
 
+// The same for the spans of one unit's gather: its cast and the peers' shards
+// on either side of it.
+constexpr int kFewSpans = 3;
+
+struct SpanFew {
+  const void* src[kFewSpans];
+  void* dst[kFewSpans];
+  int64_t numel[kFewSpans];
+  int32_t head[kFewSpans];
+  int32_t first_block[kFewSpans + 1];  // entries past the last span hold INT32_MAX
+};
+
+inline SpanFew few_runs_of(const SpanBatch& b) {
+  SpanFew f{};
+  for (int k = 0; k < kFewSpans; ++k) {
+    const bool used = k < b.count;
+    f.src[k] = used ? b.src[k] : nullptr;
+    f.dst[k] = used ? b.dst[k] : nullptr;
+    f.numel[k] = used ? b.numel[k] : 0;
+    f.head[k] = used ? b.head[k] : -1;
+  }
+  for (int k = 0; k <= kFewSpans; ++k) f.first_block[k] = k <= b.count ? b.first_block[k] : INT32_MAX;
+  return f;
+}
+
+struct SpanFewView {
+  const SpanFew& t;
+  __device__ __forceinline__ int block() const { return int(blockIdx.x); }
+  __device__ __forceinline__ SpanRun span_run(int blk) const {
+    int32_t lo = t.first_block[0], hi = t.first_block[1];
+    const void* src = t.src[0];
+    void* dst = t.dst[0];
+    int64_t numel = t.numel[0];
+    int32_t head = t.head[0];
+#pragma unroll
+    for (int k = 1; k < kFewSpans; ++k) {
+      const bool in = blk >= t.first_block[k];
+      lo = in ? t.first_block[k] : lo;
+      hi = in ? t.first_block[k + 1] : hi;
+      src = in ? t.src[k] : src;
+      dst = in ? t.dst[k] : dst;
+      numel = in ? t.numel[k] : numel;
+      head = in ? t.head[k] : head;
+    }
+    return {blk - lo, hi - lo, src, dst, numel, head};
+  }
+};
+
 struct SpanOneView {
   const SpanOne& t;
   __device__ __forceinline__ int block() const { return int(blockIdx.x); }

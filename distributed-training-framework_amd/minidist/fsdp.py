@@ -345,12 +345,16 @@ class _FSDPUnit:
         return (self.flat_shard.data_ptr(), self._full.data_ptr() + self.rank * S * self._full.element_size(), S)
 
     def _peer_slot_spans(self) -> list[tuple[int, int, int]]:
-        """(peer's gathered shard, its slot, S) for every peer (ResidentGroup): the all-gather."""
+        """(peers' gathered shards, their slots, elements) before and after this rank's (ResidentGroup):
+        the all-gather.  Both sides are rows of S elements of the gathered dtype, one after another, so
+        the peers on either side of this rank are one run."""
         self._require_gathered_storage()
-        # both are rows of S elements of the gathered dtype, one after another
-        S, step = self.shard_numel, self.shard_numel * self._full.element_size()
-        src, dst = self._peer_shards.data_ptr(), self._full.data_ptr()
-        return [(src + r * step, dst + r * step, S) for r in range(self.world) if r != self.rank]
+        S, rank, after = self.shard_numel, self.rank, self.rank + 1
+        src, dst, skip = self._peer_shards.data_ptr(), self._full.data_ptr(), after * S * self._full.element_size()
+        rows = [(src, dst, rank * S)] if rank > 0 else []
+        if after < self.world:
+            rows.append((src + skip, dst + skip, (self.world - after) * S))
+        return rows
 
     def _account_all_gather(self) -> None:
         if self.world > 1:
@@ -896,7 +900,7 @@ class FullyShardedDataParallel(nn.Module):
             by_dtype: dict[tuple[torch.dtype, torch.dtype], list] = {}
             for u in units:
                 by_dtype.setdefault((u.flat_shard.dtype, u._full.dtype), []).append(u._own_slot_span())
-            if resident and not ipc and len(by_dtype) == 1 and len(units) * self.world_size <= _KERNARG_RUNS:
+            if resident and not ipc and len(by_dtype) == 1 and 3 * len(units) <= _KERNARG_RUNS:
                 ((src, dst), casts), = by_dtype.items()
                 for u in units:
                     u._account_all_gather()

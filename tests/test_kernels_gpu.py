@@ -206,7 +206,7 @@ def test_unscale_in_place_matches_oracle(rng, dt):
 
 @pytest.mark.parametrize("sdt", DTYPES)
 @pytest.mark.parametrize("ddt", DTYPES)
-@pytest.mark.parametrize("n_casts,n_copies", [(1, 0), (1, 7), (3, 1), (8, 40), (20, 40)])
+@pytest.mark.parametrize("n_casts,n_copies", [(1, 0), (1, 2), (2, 1), (1, 7), (3, 1), (8, 40), (20, 40)])
 def test_pack_mixed_sources_matches_oracle(rng, sdt, ddt, n_casts, n_copies):
     """The first spans from one dtype and the others from the destination's, in one dispatch (up to 48
     spans) or a cast and a copy dispatch, with empty, ragged and misaligned spans and a flag clear."""
